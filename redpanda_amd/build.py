@@ -42,17 +42,6 @@ def _torch_lib_dir():
         return os.path.join(sysconfig.get_paths()["purelib"], "torch", "lib")
 
 
-# Per-file flags.  The scan backward is scheduled with LLVM's iterative ILP
-# strategy for AMDGPU: the same instructions in another order (bitwise-
-# identical results), 2 % faster at the Eval-Mamba shape and in the model's
-# configuration than the default scheduler, the same at other shapes.
-FILE_FLAGS = {
-    "scan_bwd.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"],
-    "scan_bwd_fast.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"],
-    "scan_bwd_walk.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"],
-}
-
-
 def sources(csrc=CSRC):
     return sorted(os.path.join(csrc, f) for f in os.listdir(csrc) if f.endswith(".hip"))
 
@@ -65,7 +54,7 @@ def build(verbose=False, extra_flags=(), csrc=CSRC, out=LIB_PATH):
     objs, procs = [], []
     for src in srcs:
         obj = os.path.join(tmp, os.path.basename(src) + ".o")
-        cmd = [HIPCC, *DEVICE_FLAGS, *FILE_FLAGS.get(os.path.basename(src), []), *extra_flags,
+        cmd = [HIPCC, *DEVICE_FLAGS, *extra_flags,
                "-I", INCLUDE, "-I", csrc, "-c", src, "-o", obj]
         if verbose:
             print(" ".join(cmd), flush=True)

@@ -303,7 +303,8 @@ hipError_t launch_ply_gather(const PlyGatherParams& p, hipStream_t st);
 
 // Compiled (S, NPL) shapes: S lanes per channel, NPL states per lane.
 // d_state <= 20 uses 4 lanes per channel, <= 40 uses 8, <= 128 uses 16.
-#define RP_FOR_EACH_SHAPE(X) \
+#define RP_FOR_EACH_SHAPE_4_8(X) \
   X(4, 1) X(4, 2) X(4, 3) X(4, 4) X(4, 5) \
-  X(8, 3) X(8, 4) X(8, 5) \
-  X(16, 3) X(16, 4) X(16, 5) X(16, 6) X(16, 8)
+  X(8, 3) X(8, 4) X(8, 5)
+#define RP_FOR_EACH_SHAPE_16(X) X(16, 3) X(16, 4) X(16, 5) X(16, 6) X(16, 8)
+#define RP_FOR_EACH_SHAPE(X) RP_FOR_EACH_SHAPE_4_8(X) RP_FOR_EACH_SHAPE_16(X)

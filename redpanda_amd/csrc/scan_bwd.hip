@@ -1,7 +1,7 @@
 // Launchers and reduction kernels of the scan backward, and its general
 // (non-FAST) instantiations; the kernel itself is in scan_bwd_kernel.h and its
-// whole-tile instantiations in scan_bwd_fast.hip (separate translation units
-// so that the two compile in parallel).
+// FAST instantiations in scan_bwd_fast*.hip (separate translation units, so
+// that they compile in parallel).
 
 #include "scan_bwd_kernel.h"
 
@@ -68,14 +68,12 @@ __global__ void bwd_reduce_par(const double* __restrict__ part, float* __restric
 }
 
 // Whether a launch takes the FAST instantiation: no initial state and no
-// final-state gradients, every tile's channels present, and every array the
-// chunk loop addresses spanning less than 4 GiB (its byte offsets then fit
-// in 32 bits).
-static bool bwd_fast(const ScanParams& p, const BwdIO& io, int CB) {
+// final-state gradients, and every array the chunk loop addresses spanning
+// less than 4 GiB (its byte offsets then fit in 32 bits).
+static bool bwd_fast(const ScanParams& p, const BwdIO& io) {
   if (p.h0 != nullptr || io.dh_last != nullptr || io.dbeta_last != nullptr || io.d_h0 != nullptr)
     return false;
-  if (p.D % CB != 0) return false;
-  const int64_t lim = (int64_t)1 << 32;
+  const int64_t lim = ((int64_t)1 << 32) - 4;  // a 16-bit array's base may lie 2 bytes into a word
   auto es = [](int dt) { return (int64_t)(dt == RP_F32 ? 4 : 2); };
   // one past the last byte of a (B, L, inner) array with strides sb, sl
   auto span = [&](int64_t sb, int64_t sl, int64_t inner, int64_t e) {
@@ -89,22 +87,42 @@ static bool bwd_fast(const ScanParams& p, const BwdIO& io, int CB) {
          (int64_t)p.B * p.L * p.D * 4 < lim && (half + (int64_t)p.L * p.N) * 4 < lim;
 }
 
-template <int S, int NPL, class GK>
-static hipError_t launch_bwd_t(const ScanParams& p, const BwdIO& io, hipStream_t st) {
-  dim3 grid((unsigned)((int64_t)io.ntg * io.nbg));
-  hipLaunchKernelGGL((scan_bwd_kernel<S, NPL, GK, false, false>), grid, dim3(kThreads), 0, st, p,
-                     io);
-  return hipGetLastError();
+// The FAST instantiation's types: the combinations that training hands over
+// have instantiations of their own (4 % faster at the Eval-Mamba shape than
+// reading the types at run time, 3 % in fp32), the rest share one.
+static int bwd_types(const ScanParams& p, const BwdIO& io) {
+  const int dd = p.dsp ? RP_F32 : p.dt_delta;  // delta as staged
+  const bool d32 = dd == RP_F32, u32 = p.dt_u == RP_F32;
+  const bool s32 = p.dt_B == RP_F32 && p.dt_C == RP_F32;
+  if (d32 && u32 && s32 && io.dt_dd == RP_F32 && io.dt_du == RP_F32) return kBwdF32;
+  if (d32 && !u32 && s32) return kBwdModel;
+  if (dd == RP_BF16 && p.dt_u == RP_BF16 && p.dt_B == RP_BF16 && p.dt_C == RP_BF16) return kBwdBf16;
+  return kBwdAny;
+}
+
+template <int TY>
+static hipError_t launch_fast(int S, int NPL, int gk, const ScanParams& p, const BwdIO& io,
+                              hipStream_t st) {
+  if (io.tpw > 1) return launch_scan_bwd_fast_walk<TY>(S, NPL, gk, p, io, st);
+  if (S == 16) return launch_scan_bwd_fast16<TY>(S, NPL, gk, p, io, st);
+  return launch_scan_bwd_fast<TY>(S, NPL, gk, p, io, st);
 }
 
 hipError_t launch_scan_bwd(int S, int NPL, int gk, const ScanParams& p, const BwdIO& io,
                            hipStream_t st) {
-  if (S > 0 && bwd_fast(p, io, kWaves * (kWave / S))) return launch_scan_bwd_fast(S, NPL, gk, p, io, st);
-  if (io.tpw > 1) return launch_scan_bwd_walk(S, NPL, gk, false, p, io, st);
+  if (bwd_fast(p, io)) {
+    switch (bwd_types(p, io)) {
+      case kBwdF32: return launch_fast<kBwdF32>(S, NPL, gk, p, io, st);
+      case kBwdBf16: return launch_fast<kBwdBf16>(S, NPL, gk, p, io, st);
+      case kBwdModel: return launch_fast<kBwdModel>(S, NPL, gk, p, io, st);
+      default: return launch_fast<kBwdAny>(S, NPL, gk, p, io, st);
+    }
+  }
+  if (io.tpw > 1) return launch_scan_bwd_walk(S, NPL, gk, p, io, st);
 #define RP_CASE(SS, NN)                                                              \
   if (S == SS && NN == NPL)                                                          \
     return with_gate_kind_scan<SS, NN>(gk, [&](auto g) {                                      \
-      return launch_bwd_t<SS, NN, decltype(g)>(p, io, st);                           \
+      return launch_bwd_kernel<SS, NN, decltype(g), false, false, kBwdAny>(p, io, st); \
     });
   RP_FOR_EACH_SHAPE(RP_CASE)
 #undef RP_CASE

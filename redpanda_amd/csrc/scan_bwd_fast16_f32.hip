@@ -1,0 +1,6 @@
+// The scan backward's FAST instantiations: 16-lane shapes, fp32 inputs and outputs.
+#include "scan_bwd_fast_inst.h"
+
+namespace rp {
+template hipError_t launch_scan_bwd_fast16<kBwdF32>(int, int, int, const ScanParams&, const BwdIO&, hipStream_t);
+}

@@ -1,0 +1,6 @@
+// The scan backward's FAST instantiations: 16-lane shapes, tile walk, the model's storage types.
+#include "scan_bwd_fast_inst.h"
+
+namespace rp {
+template hipError_t launch_scan_bwd_fast_walk<kBwdModel>(int, int, int, const ScanParams&, const BwdIO&, hipStream_t);
+}

@@ -24,10 +24,10 @@
 // the backward walks chunks in reverse, recomputes the chunk's K steps into
 // registers (keeping s_{t-1}, the gate and e*sin, so the adjoint evaluates
 // no transcendental), then runs the adjoint over them.  The recompute
-// evaluates the forward's gate expansion from (m, b sin) table records,
-// which also give the sine (one 8-byte table read; the forward's records
-// would need a second read for it); each gate matches the forward's to
-// within an ulp and every chunk restarts from the forward's checkpoint.
+// takes each gate and its sine from a finer table than the forward's (one
+// 8-byte read, a quadratic and its derivative: rp_device.h); each gate
+// matches the forward's to within an ulp and every chunk restarts from the
+// forward's checkpoint.
 //
 // Streaming: the per-step inputs (dt, (dt*u)/2, u, dy per channel; B, C per
 // state) of a chunk and of the step before it sit in one of two LDS slots.
@@ -40,8 +40,8 @@
 //
 // Reductions, all in a fixed order (run-to-run deterministic; no address is
 // updated by more than one thread):
-//   * over a channel's states (ddt, du): in-lane FMA chain, then the S lanes'
-//     partials summed pairwise from LDS where the chunk's outputs are written;
+//   * over a channel's states (ddt, du): in-lane FMA chain and lane pairs, then
+//     the pairs' partials summed from LDS where the chunk's outputs are written;
 //   * over channels (dB, dC): DPP row rotations inside each 16-lane row, the
 //     row partials staged in LDS, then a balanced 16-way sum per output, per tile;
 //     the per-tile partials are summed in float64 by a second kernel;
@@ -63,9 +63,18 @@ namespace rp {
 // added into the float64 sums (64 steps).
 constexpr int kParChunks = 16;
 
-// FAST: the instantiation for launches with no initial state, no final-state
-// gradients and every channel of every tile present, whose arrays span less
-// than 4 GiB each (bwd_fast in scan_bwd.hip).  Every global address of the chunk loop
+// How a FAST instantiation knows the storage types of its inputs and outputs.
+enum BwdTypes {
+  kBwdAny = 0,    // any mix, read at run time
+  kBwdF32 = 1,    // delta as staged, u, B, C and both outputs in fp32
+  kBwdBf16 = 2,   // delta as staged, u, B and C in bf16
+  kBwdModel = 3,  // u in bf16 or fp16; delta as staged (the forward's softplus
+                  // cache), B and C in fp32 (the model under autocast)
+};
+
+// FAST: the instantiation for launches with no initial state and no
+// final-state gradients, whose arrays span less than 4 GiB each (bwd_fast in
+// scan_bwd.hip).  Every global address of the chunk loop
 // is then a wave-uniform base pointer plus a 32-bit byte offset, taken per
 // batch-row sweep and moved by a uniform multiple of the chunk index: one
 // full-rate add per staged element, where the general form multiplies 64-bit
@@ -76,7 +85,8 @@ constexpr int kParChunks = 16;
 // tgrp), batch group bgi.  The tiles of a group share one dB / dC partial
 // block: the first writes it, the others add onto it (as the reverse
 // direction adds onto the forward direction's), in tile order.
-template <int S, int NPL, class GK, bool FAST, bool MULTI>
+// TY: the storage types of a FAST launch (BwdTypes).
+template <int S, int NPL, class GK, bool FAST, bool MULTI, int TY>
 __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& io, int tile,
                                               int tpass, int tgrp, int bgi) {
   using Sh = Shape<S, NPL>;
@@ -116,10 +126,12 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
   constexpr bool PAR_GLOBAL = (S * NPL > 40 && FOLD_CHUNK) || ONEBAR;
   constexpr int NFOLD = K / KR;             // folds per chunk
   constexpr int NRW = kWaves * 4;           // 16-lane rows per workgroup
-  // row partials of one output are contiguous (4 x 16-byte reads); the
-  // padding to 20 spreads the writers of a row over distinct banks
-  constexpr int RWP = NRW + 4;
   static_assert(NRW == 16, "the fold sums 16 row partials");
+  // Row partials of one output (state n) are contiguous, one 16-byte quad
+  // per wave; the quads are permuted by an XOR with rho(n), so that a wave's
+  // writes (16 lanes' states, 4 rows) and a reader's 16-byte quads of
+  // adjacent states meet distinct banks without padding.
+  auto rho = [](int n) { return (n >> 2) & (S == 16 ? 3 : 1); };
   constexpr int FPT = (KR * 2 * NP + kThreads - 1) / kThreads;  // fold outputs per thread
   constexpr int KS = K + 1;  // staged steps per chunk: the step before it, then its K steps
   constexpr int CPT = (KS * CB + kThreads - 1) / kThreads;      // staged channel-steps per thread
@@ -130,17 +142,19 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
   constexpr bool KEEP_HT = NP <= 40;
   static_assert(K % KR == 0, "a chunk holds whole folds");
   __shared__ float4 sCh[2][KS][CB];       // input slots: (dt, (dt*u)/2, u/2, dy)
-  __shared__ float sB[2][KS][NP];
-  __shared__ float sC[2][KS][NP];
-  __shared__ __align__(16) float sRed[NB][KR][2][NP][RWP];  // per-row channel sums of dB, dC
+  // (B, C) pairs: one 8-byte access each, whose 16-bit offsets reach the
+  // whole slot (4-byte pairs of two arrays needed address arithmetic)
+  __shared__ float2 sBC[2][KS][NP];
+  __shared__ __align__(16) float sRed[NB][KR][2][NP][NRW];  // per-row channel sums of dB, dC
   // per lane: its (d gate / d dt, dhb . B) sums over its states of each
-  // chunk step, summed over the channel's S lanes where the chunk's
-  // (d_delta, d_u) are written.  Channel-contiguous per lane slice s; the
-  // row of a slice padded to CB + 16/S so that 16 lanes' writes (16/S
-  // channels x S slices) meet 32 distinct banks.
-  constexpr int DDP = CB + 16 / S;
-  __shared__ float2 sDD[NB][K][S][DDP];
-  __shared__ float2 sCS[kTab];              // (m, b sin) records of the gate table
+  // chunk step, added in pairs of adjacent lanes and summed over the
+  // channel's S / 2 pairs where the chunk's (d_delta, d_u) are written.
+  // Channel-contiguous per pair; a pair's row padded to CB + DT so that a
+  // wave's 32 distinct writes (DT channels x S / 2 pairs) meet distinct banks.
+  constexpr int SP2 = S / 2, DDP = CB + DT;
+  __shared__ float2 sDD[NB][K][SP2][DDP];
+  // (m, b (-s a)) records of the backward's gate table (none for real decay)
+  __shared__ float2 sCS[GK::kImag == 0 ? 1 : kTabB];
   // per-thread float64 sums of the parameter gradients over the batch group
   // (dA_real or dtrack, dA_imag), kept in LDS to spare registers (in their
   // global partials when PAR_GLOBAL)
@@ -154,9 +168,8 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
   const int wave = tid / kWave, lane = tid % kWave;
   const int dl = lane / S, s = lane % S;
   const int cl = wave * DT + dl;
-  const int wrow = wave * 4 + lane / 16;  // row index within the workgroup
   const int c = tile * CB + cl;
-  const bool cvalid = FAST || c < p.D;
+  const bool cvalid = c < p.D;
   const bool has_imag = p.Ai != nullptr;
   const int L = p.L;
 
@@ -164,16 +177,21 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
   load_gate_regs<S, NPL>(gp, p.Ar, p.Ai, p.Tk, c, s, p.N, p.NR, p.NT, cvalid);
   // first read after the staging barrier below (the table stays from the
   // workgroup's first tile on)
-  if (tpass == 0) fill_sincos_pairs(sCS, tid);
+  if (GK::kImag != 0 && tpass == 0) fill_sincos_fine(sCS, tid);
   // pam: the coefficient of the ddt sum over rotational states, zero for a
   // tracking state (only read for slots whose kind is decided at run time)
   float pam[NPL];
+  // where this lane's row partials go within a (step, dB or dC) block: state
+  // j S + s at j S * NRW beyond it (at 4 lanes rho alternates with j)
+  const int wofs = s * NRW + ((wave ^ rho(s)) * 4 + (lane >> 4));
+  const int wofs1 = S == 4 ? s * NRW + ((wave ^ 1) * 4 + (lane >> 4)) : wofs;
   // this thread's entry for state slot j of the per-batch-group partials
   // (dA_real or dtrack; dA_imag is one D*N block further)
   auto par_at = [&](int j) { return ((int64_t)bgi * 2) * p.D * p.N + (int64_t)c * p.N + j * S + s; };
 #pragma unroll
   for (int j = 0; j < NPL; ++j) {
     pam[j] = is_rot<S, GK>(j, s, p.NR) ? gp.pah[j] : 0.f;
+    gp.wh[j] *= (float)(kTabB / kTab);  // in the backward table's steps
     if constexpr (PAR_GLOBAL) {
       if (cvalid && j * S + s < p.N) {
         io.part_par[par_at(j)] = 0.0;
@@ -199,6 +217,11 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
   const int64_t d_sb = cached ? (int64_t)L * p.D : p.dsb;
   const int64_t d_sl = cached ? (int64_t)p.D : p.dsl;
   const int d_dt = cached ? RP_F32 : p.dt_delta;
+  // FAST, types not fixed: a 16-bit array's offset from the 32-bit word that
+  // its base lies in
+  auto word_off = [](const void* q) {
+    return TY == kBwdAny ? (uint32_t)(reinterpret_cast<uintptr_t>(q) & 3) : 0u;
+  };
   // FAST: this thread's byte offsets for the sweep (b, dir) as they would be
   // at chunk 0, and the wave-uniform byte step per chunk: the offset at chunk
   // ch is o + ch * step (mod 2^32; the elements a lane loads or stores lie in
@@ -206,9 +229,12 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
   // sweep's (tile group, b) block of the dB / dC partials, pbc.
   uint32_t oDT[CPT], oU[CPT], oDY[CPT], oB[SPT], oC[SPT], oF[NFOLD][FPT], oD[DPT];
   uint32_t stDT = 0, stU = 0, stDY = 0, stB = 0, stC = 0, stF = 0;
+  // FAST: whether element k of this thread's channel-steps and state-steps
+  // exists (its place in the slot, its channel or state)
+  bool okC[CPT], okS[SPT], okD[DPT];
   float* pbc = io.part_bc;
-  // FAST: fold output k of this thread as LDS float index * 8 + its row
-  // within the fold, or -1 beyond the fold's outputs
+  // FAST: fold output k of this thread as the LDS quad index of its wave-0
+  // partials * 8 + its row within the fold, or -1 beyond the fold's outputs
   int fInfo[FPT];
   // FAST: fold output of this thread in round k; the last, partial round
   // runs on the last waves (the d_delta / d_u outputs run on the first)
@@ -225,8 +251,7 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
       if (e >= 0 && e < KR * 2 * p.N) {
         const int rr = e / (2 * p.N), rem = e % (2 * p.N);
         const int which = rem / p.N, n = rem % p.N;
-        const int kk = (n % S) * NPL + n / S;
-        fInfo[k] = (((rr * 2 + which) * NP + kk) * RWP) * 8 + rr;
+        fInfo[k] = (((rr * 2 + which) * NP + n) * (NRW / 4) + rho(n)) * 8 + rr;
       }
     }
   }
@@ -239,8 +264,9 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
     for (int k = 0; k < CPT; ++k) {
       const int e = tid + k * kThreads;
       const int64_t t = t0 + sg * (e / CB - 1), c2 = tile * CB + e % CB;
-      oDT[k] = (uint32_t)((b * d_sb + t * d_sl + c2) * es_d);
-      oU[k] = (uint32_t)((b * p.usb + t * p.usl + c2) * es_u);
+      okC[k] = e < KS * CB && c2 < p.D;
+      oDT[k] = (uint32_t)((b * d_sb + t * d_sl + c2) * es_d) + word_off(dsrc);
+      oU[k] = (uint32_t)((b * p.usb + t * p.usl + c2) * es_u) + word_off(p.u);
       oDY[k] = (uint32_t)((((int64_t)b * L + t) * p.D + c2) * 4);
     }
 #pragma unroll
@@ -248,8 +274,9 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
       const int e = tid + k * kThreads;
       const int kk = e % NP;
       const int64_t t = t0 + sg * (e / NP - 1), n = (kk % NPL) * S + kk / NPL;
-      oB[k] = (uint32_t)((b * p.bsb + t * p.bsl + n) * es_b);
-      oC[k] = (uint32_t)((b * p.csb + t * p.csl + n) * es_c);
+      okS[k] = e < KS * NP && n < p.N;
+      oB[k] = (uint32_t)((b * p.bsb + t * p.bsl + n) * es_b) + word_off(p.Bc);
+      oC[k] = (uint32_t)((b * p.csb + t * p.csl + n) * es_c) + word_off(p.Cc);
     }
     const int64_t half = (int64_t)io.ntg * p.B * L * p.N;  // the dC half of the partials
 #pragma unroll
@@ -266,6 +293,7 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
     for (int k = 0; k < DPT; ++k) {
       const int e = tid + k * kThreads;
       const int64_t t = t0 + sg * (e / CB), c2 = tile * CB + e % CB;
+      okD[k] = e < K * CB && c2 < p.D;
       oD[k] = (uint32_t)((((int64_t)b * L + t) * p.D + c2) * 4);
     }
     stDT = (uint32_t)(sg * K * d_sl * es_d);
@@ -276,78 +304,62 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
     stF = (uint32_t)(sg * K * p.N * 4);
     pbc = io.part_bc + ((int64_t)tgrp * p.B + b) * L * p.N;
   };
-  // FAST: the storage codes of (delta as staged, u, B and C) as one of the
-  // common combinations, fixed at compile time in the staging code, so that
-  // a staging branches once on them instead of once per element (-1: codes
-  // read at run time)
-  const int tcombo =
-      !FAST ? -1
-      : (d_dt == RP_BF16 && p.dt_u == RP_BF16 && p.dt_B == RP_BF16 && p.dt_C == RP_BF16) ? 0
-      : (d_dt == RP_F32 && p.dt_u == RP_F32 && p.dt_B == RP_F32 && p.dt_C == RP_F32)     ? 1
-      : (d_dt == RP_F32 && p.dt_u == RP_BF16 && p.dt_B == RP_F32 && p.dt_C == RP_F32)    ? 2
-      : (d_dt == RP_F32 && p.dt_u == RP_F16 && p.dt_B == RP_F32 && p.dt_C == RP_F32)     ? 3
-      : (d_dt == RP_F16 && p.dt_u == RP_F16 && p.dt_B == RP_F16 && p.dt_C == RP_F16)     ? 4
-                                                                                          : -1;
-  using TBF = std::integral_constant<int, RP_BF16>;
-  using TF32 = std::integral_constant<int, RP_F32>;
-  using TF16 = std::integral_constant<int, RP_F16>;
-  using TRT = std::integral_constant<int, -1>;
-  auto with_types = [&](auto f) {
-    switch (tcombo) {
-      case 0: f(TBF{}, TBF{}, TBF{}); break;
-      case 1: f(TF32{}, TF32{}, TF32{}); break;
-      case 2: f(TF32{}, TBF{}, TF32{}); break;
-      case 3: f(TF32{}, TF16{}, TF32{}); break;
-      case 4: f(TF16{}, TF16{}, TF16{}); break;
-      default: f(TRT{}, TRT{}, TRT{}); break;
-    }
-  };
-  // an element as stored (type IT, or the run-time code rt when IT is -1),
-  // and its value
-  auto load_t = [&](auto it_tag, const void* base, uint32_t off, int rt) -> uint32_t {
-    constexpr int IT = decltype(it_tag)::value;
-    if constexpr (IT < 0)
-      return load_raw_byte(base, off, rt);
+  // FAST: the storage widths of delta (as staged), u and B / C, fixed by TY
+  // (0: any).  In kBwdModel bf16 and fp16 are told apart by a select.
+  constexpr int WD = TY == kBwdF32 || TY == kBwdModel ? 32 : TY == kBwdBf16 ? 16 : 0;
+  constexpr int WU = TY == kBwdF32 ? 32 : TY == kBwdAny ? 0 : 16;
+  // Width 0 needs no branch on the storage type either: the aligned 32-bit
+  // word that holds the element is loaded (at most its other half lies outside
+  // the array, never another word), and where it is staged the element
+  // is rotated to the word's low half by its byte offset (which keeps its
+  // place in the word from chunk to chunk: K steps are a multiple of 8 bytes)
+  // and shifted or converted.  A switch over the types' combinations cost its
+  // branches, and their joins' waits, in every chunk: at the Eval-Mamba shape
+  // 2.47 ms, 2.38 with words, 2.28 with the widths fixed.
+  using WDT = std::integral_constant<int, WD>;
+  using WUT = std::integral_constant<int, WU>;
+  auto load_el = [&](auto w_tag, const void* base, uint32_t off) -> uint32_t {
+    constexpr int W = decltype(w_tag)::value;
+    if constexpr (W == 32)
+      return load_byte<uint32_t>(base, off);
+    else if constexpr (W == 16)
+      return load_byte<uint16_t>(base, off);
     else
-      return load_byte<RawOf<IT>>(base, off);
+      return load_byte<uint32_t>(static_cast<const char*>(base) - word_off(base), off & ~3u);
   };
-  auto cvt_t = [&](auto it_tag, uint32_t v, int rt) -> float {
-    constexpr int IT = decltype(it_tag)::value;
-    if constexpr (IT < 0)
-      return cvt_raw(v, rt);
-    else
-      return cvt_raw(v, IT);
+  auto el_value = [&](auto w_tag, uint32_t w, uint32_t off, int dt) -> float {
+    constexpr int W = decltype(w_tag)::value;
+    if constexpr (W == 32) return __uint_as_float(w);
+    const uint32_t v = W == 16 ? w : __builtin_amdgcn_alignbyte(w, w, off);
+    const float f = __uint_as_float(W == 0 && dt == RP_F32 ? v : v << 16);
+    const float h = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(v)));
+    return TY != kBwdBf16 && dt == RP_F16 ? h : f;
   };
   auto stage_load = [&](int b, int dir, int ch) {
     if constexpr (FAST) {
       const uint32_t cu = (uint32_t)ch;
-      with_types([&](auto tdt, auto tu, auto ts) {
 #pragma unroll
-        for (int k = 0; k < CPT; ++k) {
-          const int e = tid + k * kThreads;
-          const int i = ch * K + e / CB - 1;
-          rdt[k] = 0u;
-          ru[k] = 0u;
-          rdy[k] = 0.f;
-          if (e < KS * CB && (unsigned)i < (unsigned)L) {
-            rdt[k] = load_t(tdt, dsrc, oDT[k] + cu * stDT, d_dt);
-            ru[k] = load_t(tu, p.u, oU[k] + cu * stU, p.dt_u);
-            rdy[k] = load_byte<float>(io.dy, oDY[k] + cu * stDY);
-          }
+      for (int k = 0; k < CPT; ++k) {
+        const int i = ch * K + (tid + k * kThreads) / CB - 1;
+        rdt[k] = 0u;
+        ru[k] = 0u;
+        rdy[k] = 0.f;
+        if (okC[k] && (unsigned)i < (unsigned)L) {
+          rdt[k] = load_el(WDT{}, dsrc, oDT[k] + cu * stDT);
+          ru[k] = load_el(WUT{}, p.u, oU[k] + cu * stU);
+          rdy[k] = load_byte<float>(io.dy, oDY[k] + cu * stDY);
         }
+      }
 #pragma unroll
-        for (int k = 0; k < SPT; ++k) {
-          const int e = tid + k * kThreads;
-          const int kk = e % NP;
-          const int i = ch * K + e / NP - 1;
-          rb[k] = 0u;
-          rc[k] = 0u;
-          if (e < KS * NP && (kk % NPL) * S + kk / NPL < p.N && (unsigned)i < (unsigned)L) {
-            rb[k] = load_t(ts, p.Bc, oB[k] + cu * stB, p.dt_B);
-            rc[k] = load_t(ts, p.Cc, oC[k] + cu * stC, p.dt_C);
-          }
+      for (int k = 0; k < SPT; ++k) {
+        const int i = ch * K + (tid + k * kThreads) / NP - 1;
+        rb[k] = 0u;
+        rc[k] = 0u;
+        if (okS[k] && (unsigned)i < (unsigned)L) {
+          rb[k] = load_el(WDT{}, p.Bc, oB[k] + cu * stB);
+          rc[k] = load_el(WDT{}, p.Cc, oC[k] + cu * stC);
         }
-      });
+      }
       return;
     }
 #pragma unroll
@@ -383,25 +395,22 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
   auto stage_store = [&](auto slot_tag) {
     constexpr int SL = decltype(slot_tag)::value;
     if constexpr (FAST) {
-      with_types([&](auto tdt, auto tu, auto ts) {
 #pragma unroll
-        for (int k = 0; k < CPT; ++k) {
-          const int e = tid + k * kThreads;
-          if (e < KS * CB) {
-            const float dt = cvt_t(tdt, rdt[k], d_dt);
-            const float uu = cvt_t(tu, ru[k], p.dt_u);
-            sCh[SL][e / CB][e % CB] = make_float4(dt, 0.5f * fmul(dt, uu), 0.5f * uu, rdy[k]);
-          }
+      for (int k = 0; k < CPT; ++k) {
+        const int e = tid + k * kThreads;
+        if (e < KS * CB) {
+          const float dt = el_value(WDT{}, rdt[k], oDT[k], d_dt);
+          const float uu = el_value(WUT{}, ru[k], oU[k], p.dt_u);
+          sCh[SL][e / CB][e % CB] = make_float4(dt, 0.5f * fmul(dt, uu), 0.5f * uu, rdy[k]);
         }
+      }
 #pragma unroll
-        for (int k = 0; k < SPT; ++k) {
-          const int e = tid + k * kThreads;
-          if (e < KS * NP) {
-            sB[SL][e / NP][e % NP] = cvt_t(ts, rb[k], p.dt_B);
-            sC[SL][e / NP][e % NP] = cvt_t(ts, rc[k], p.dt_C);
-          }
-        }
-      });
+      for (int k = 0; k < SPT; ++k) {
+        const int e = tid + k * kThreads;
+        if (e < KS * NP)
+          sBC[SL][e / NP][e % NP] =
+              make_float2(el_value(WDT{}, rb[k], oB[k], p.dt_B), el_value(WDT{}, rc[k], oC[k], p.dt_C));
+      }
       return;
     }
 #pragma unroll
@@ -417,8 +426,7 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
     for (int k = 0; k < SPT; ++k) {
       const int e = tid + k * kThreads;
       if (e < KS * NP) {
-        sB[SL][e / NP][e % NP] = cvt_raw(rb[k], p.dt_B);
-        sC[SL][e / NP][e % NP] = cvt_raw(rc[k], p.dt_C);
+        sBC[SL][e / NP][e % NP] = make_float2(cvt_raw(rb[k], p.dt_B), cvt_raw(rc[k], p.dt_C));
       }
     }
   };
@@ -474,18 +482,18 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
     if (e >= K * CB || r >= kcnt || c2 >= p.D) return -1;
     return ((int64_t)b * L + tix(dir, i0 + r)) * p.D + c2;
   };
-  // (d_delta, d_u) of one chunk step and channel from its S lanes' partial
+  // (d_delta, d_u) of one chunk step and channel from its lane pairs' partial
   // sums (d gate / d dt, dhb . B) in sDD: the sums over the lanes in the
   // order of reduce_states (pairwise, adjacent halves), then
   //     d_delta = dga + u/2 * sBc,   d_u = dt/2 * sBc   (hb = (dt*u)/2 * B)
   auto dd_of = [&](int buf, int r, int cc, float dt, float uh) -> float2 {
-    float2 v[S];
+    float2 v[SP2];
 #pragma unroll
-    for (int i = 0; i < S; ++i) v[i] = sDD[buf][r][i][cc];
+    for (int i = 0; i < SP2; ++i) v[i] = sDD[buf][r][i][cc];
 #pragma unroll
-    for (int w = 1; w < S; w *= 2)
+    for (int w = 1; w < SP2; w *= 2)
 #pragma unroll
-      for (int i = 0; i < S; i += 2 * w) v[i] = make_float2(v[i].x + v[i + w].x, v[i].y + v[i + w].y);
+      for (int i = 0; i < SP2; i += 2 * w) v[i] = make_float2(v[i].x + v[i + w].x, v[i].y + v[i + w].y);
     return make_float2(v[0].x + fmul(uh, v[0].y), fmul(0.5f * dt, v[0].y));
   };
   // whether this direction's d_delta store is the last one (the gradient
@@ -565,6 +573,7 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
 
       // one chunk, its slot and whether it is whole fixed at compile time
       auto one_chunk = [&](const int ch, auto full_arg, auto slot_arg) {
+        constexpr bool FULLC = decltype(full_arg)::value;
         const int i0 = ch * K;
         const int kcnt = min(K, L - i0);
         float prev[NFOLD][FPT], pdd[DPT][2];
@@ -581,7 +590,7 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
             for (int k = 0; k < FPT; ++k) {
               prev[f][k] = 0.f;
               if constexpr (FAST) {
-                if (add_bc && fInfo[k] >= 0 && f * KR + (fInfo[k] & 7) < kcnt)
+                if (add_bc && fInfo[k] >= 0 && (FULLC || f * KR + (fInfo[k] & 7) < kcnt))
                   prev[f][k] = load_byte<float>(pbc, oF[f][k] + (uint32_t)ch * stF);
               } else if (add_bc) {
                 const float* src = fold_dst(tid + k * kThreads, b, dir, i0, f * KR, kcnt);
@@ -594,8 +603,7 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
             pdd[k][0] = 0.f;
             pdd[k][1] = 0.f;
             if constexpr (FAST) {
-              const int e = tid + k * kThreads;
-              if (dir == 1 && e < K * CB && e / CB < kcnt) {
+              if (dir == 1 && okD[k] && (FULLC || (tid + k * kThreads) / CB < kcnt)) {
                 const uint32_t o = oD[k] + (uint32_t)ch * stDY;
                 pdd[k][0] = load_byte<float>(io.pd_delta, o);
                 pdd[k][1] = load_byte<float>(io.pd_u, o);
@@ -652,7 +660,7 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
           } else {
             const float hdp = sCh[SL][0][cl].y;
 #pragma unroll
-            for (int j = 0; j < NPL; ++j) hbp[j] = fmul(hdp, sB[SL][0][s * NPL + j]);
+            for (int j = 0; j < NPL; ++j) hbp[j] = fmul(hdp, sBC[SL][0][s * NPL + j].x);
           }
           // recompute the chunk: s_{t-1}, g_t, e*sin and h_t for every step
           float SP[K][NPL], G[K][NPL], ES[K][NPL], HT[KEEP_HT ? K : 1][NPL];
@@ -670,7 +678,7 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
               for (int j = 0; j < NPL; ++j) {
                 float es;
                 const float g = gate_finish_cs<S, GK>(j, s, p.NR, has_imag, part[j], gp.pah[j], es);
-                const float hb = fmul(hd, sB[SL][m + 1][s * NPL + j]);
+                const float hb = fmul(hd, sBC[SL][m + 1][s * NPL + j].x);
                 const float sm = hc[j] + hbp[j];
                 SP[m][j] = sm;
                 G[m][j] = g;
@@ -697,8 +705,8 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
               float ddA = 0.f, ddB = 0.f, sBc = 0.f;
 #pragma unroll
               for (int j = 0; j < NPL; ++j) {
-                const float Bv = sB[SL][m + 1][s * NPL + j];
-                const float Cv = sC[SL][m + 1][s * NPL + j];
+                const float2 bc = sBC[SL][m + 1][s * NPL + j];
+                const float Bv = bc.x, Cv = bc.y;
                 const float g = G[m][j];
                 float ht;
                 if constexpr (KEEP_HT)
@@ -724,19 +732,22 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
                   cpb[j] = ffma(t2, dt, cpb[j]);
                   if (j >= GK::kRJ) cpt[j] = cpt[j] + dg;
                   ddA = ffma(j < GK::kRJ ? gp.pah[j] : pam[j], t1, ddA);  // Ar log2(e) dg g
-                  ddB = ffma(gp.wh[j], t2, ddB);                          // Ai 256/(2 pi) dg e sin
+                  ddB = ffma(gp.wh[j], t2, ddB);                          // -Ai dg e sin
                 }
                 qn[j] = q;
                 gn[j] = g;
                 // every lane of the row holds the row's total for its slice
                 // s, so the lanes sharing s store the same value
-                sRed[ONEBAR ? SL : 0][m % KR][0][s * NPL + j][wrow] = reduce_row<S>(fmul(dhb, hd));
-                sRed[ONEBAR ? SL : 0][m % KR][1][s * NPL + j][wrow] = reduce_row<S>(fmul(dy, ht));
+                const int wo = j % 2 ? wofs1 : wofs;
+                (&sRed[ONEBAR ? SL : 0][m % KR][0][j * S][0])[wo] = reduce_row<S>(fmul(dhb, hd));
+                (&sRed[ONEBAR ? SL : 0][m % KR][1][j * S][0])[wo] = reduce_row<S>(fmul(dy, ht));
               }
-              // d(gate)/d(dt) and sBc summed over the lane's states; their
-              // sums over the channel's lanes are taken from sDD at the
-              // chunk's end
-              sDD[ONEBAR ? SL : 0][m][s][cl] = make_float2(ffma(kLn2, ddA, -fmul(kRadPerStep, ddB)), sBc);
+              // d(gate)/d(dt) and sBc summed over the lane's states and its
+              // neighbour's (both lanes of a pair store the same sums); the
+              // rest of the sums over the channel's lanes are taken from sDD
+              // at the chunk's end
+              sDD[ONEBAR ? SL : 0][m][s / 2][cl] =
+                  make_float2(reduce_states<2>(ffma(kLn2, ddA, ddB)), reduce_states<2>(sBc));
               if constexpr (!FAST) fin = false;
             }
             if (m % KR == 0) {
@@ -790,9 +801,9 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
               for (int k = 0; k < FPT; ++k) {
                 if constexpr (FAST) {
                   if (fInfo[k] >= 0 && (FULL || m + (fInfo[k] & 7) < kcnt)) {
-                    const float4* rp =
-                        reinterpret_cast<const float4*>(&sRed[ONEBAR ? SL : 0][0][0][0][0] + (fInfo[k] >> 3));
-                    const float4 a0 = rp[0], a1 = rp[1], a2 = rp[2], a3 = rp[3];
+                    const float4* rp = reinterpret_cast<const float4*>(&sRed[ONEBAR ? SL : 0][0][0][0][0]);
+                    const int q = fInfo[k] >> 3;
+                    const float4 a0 = rp[q], a1 = rp[q ^ 1], a2 = rp[q ^ 2], a3 = rp[q ^ 3];
                     const float v = (((a0.x + a0.y) + (a0.z + a0.w)) + ((a1.x + a1.y) + (a1.z + a1.w))) +
                                     (((a2.x + a2.y) + (a2.z + a2.w)) + ((a3.x + a3.y) + (a3.z + a3.w)));
                     store_byte<float>(pbc, oF[m / KR][k] + (uint32_t)ch * stF,
@@ -805,9 +816,9 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
                 if (dst != nullptr) {
                   const int rem = e % (2 * p.N);
                   const int which = rem / p.N, n = rem % p.N;
-                  const int kk = (n % S) * NPL + n / S;
-                  const float4* rp = reinterpret_cast<const float4*>(&sRed[0][e / (2 * p.N)][which][kk][0]);
-                  const float4 a0 = rp[0], a1 = rp[1], a2 = rp[2], a3 = rp[3];
+                  const float4* rp = reinterpret_cast<const float4*>(&sRed[0][e / (2 * p.N)][which][n][0]);
+                  const int q = rho(n);
+                  const float4 a0 = rp[q], a1 = rp[q ^ 1], a2 = rp[q ^ 2], a3 = rp[q ^ 3];
                   const float v = (((a0.x + a0.y) + (a0.z + a0.w)) + ((a1.x + a1.y) + (a1.z + a1.w))) +
                                   (((a2.x + a2.y) + (a2.z + a2.w)) + ((a3.x + a3.y) + (a3.z + a3.w)));
                   *dst = add_bc ? prev[m / KR][k] + v : v;
@@ -819,15 +830,15 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
                 for (int k = 0; k < DPT; ++k) {
                   const int e = tid + k * kThreads;
                   if constexpr (FAST) {
-                    if (e < K * CB && (FULL || e / CB < kcnt)) {
+                    if (okD[k] && (FULL || e / CB < kcnt)) {
                       const uint32_t o = oD[k] + (uint32_t)ch * stDY;
                       const float2 v = dd_of(ONEBAR ? SL : 0, e / CB, e % CB, fdt[k], fuh[k]);
                       float dd = dir == 0 ? v.x : pdd[k][0] + v.x;
                       if (p.dsp && dd_final(dir)) dd = fmul(dd, fsp[k]);
                       const float du = dir == 0 ? v.y : pdd[k][1] + v.y;
                       if (dd_final(dir)) {
-                        store_grad(io.d_delta, o, dd, io.dt_dd);
-                        store_grad(io.d_u, o, du, io.dt_du);
+                        store_grad(io.d_delta, o, dd, TY == kBwdF32 ? RP_F32 : io.dt_dd);
+                        store_grad(io.d_u, o, du, TY == kBwdF32 ? RP_F32 : io.dt_du);
                       } else {
                         store_byte<float>(io.pd_delta, o, dd);
                         store_byte<float>(io.pd_u, o, du);
@@ -870,11 +881,12 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
                 if (cvalid && j * S + s < p.N) {
                   unsafeAtomicAdd(&io.part_par[par_at(j)], (double)a);
                   if (j < GK::kTJ)
-                    unsafeAtomicAdd(&io.part_par[par_at(j) + (int64_t)p.D * p.N], (double)cpb[j]);
+                    unsafeAtomicAdd(&io.part_par[par_at(j) + (int64_t)p.D * p.N],
+                                    (double)cpb[j] * kInvStepB);
                 }
               } else {
                 sPar[0][j][tid] += (double)a;
-                if (j < GK::kTJ) sPar[1][j][tid] += (double)cpb[j];
+                if (j < GK::kTJ) sPar[1][j][tid] += (double)cpb[j] * kInvStepB;
               }
               cpa[j] = 0.f;
               cpb[j] = 0.f;
@@ -957,26 +969,41 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
 // partials to write and reduce where tiles are narrow: 16 channels at 16
 // lanes); otherwise one tile (io.tpw == 1), without the loop, whose
 // hoisting would cost registers.
-template <int S, int NPL, class GK, bool FAST, bool MULTI>
+template <int S, int NPL, class GK, bool FAST, bool MULTI, int TY>
 __global__ __launch_bounds__(kThreads, NPL <= 5 ? 2 : 1) void scan_bwd_kernel(ScanParams p, BwdIO io) {
   const int tgrp = blockIdx.x % io.ntg, bgi = blockIdx.x / io.ntg;
   if constexpr (MULTI) {
     for (int tp = 0; tp < io.tpw; ++tp) {
       const int tile = tgrp * io.tpw + tp;
       if (tile >= p.ntiles) break;
-      scan_bwd_tile<S, NPL, GK, FAST, true>(p, io, tile, tp, tgrp, bgi);
+      scan_bwd_tile<S, NPL, GK, FAST, true, TY>(p, io, tile, tp, tgrp, bgi);
     }
   } else {
-    scan_bwd_tile<S, NPL, GK, FAST, false>(p, io, tgrp, 0, tgrp, bgi);
+    scan_bwd_tile<S, NPL, GK, FAST, false, TY>(p, io, tgrp, 0, tgrp, bgi);
   }
 }
 
-// The whole-tile (FAST) launches, instantiated in scan_bwd_fast.hip.
+// The FAST launches of one BwdTypes, for the 4- and 8-lane shapes, the
+// 16-lane shapes and the 16-lane shapes' tile walk (MULTI: io.tpw > 1).
+template <int TY>
 hipError_t launch_scan_bwd_fast(int S, int NPL, int gk, const ScanParams& p, const BwdIO& io,
                                 hipStream_t st);
-// The tile-walking (MULTI) launches of the 16-lane shapes, whole-tile or
-// general, instantiated in scan_bwd_walk.hip.
-hipError_t launch_scan_bwd_walk(int S, int NPL, int gk, bool fast, const ScanParams& p,
-                                const BwdIO& io, hipStream_t st);
+template <int TY>
+hipError_t launch_scan_bwd_fast16(int S, int NPL, int gk, const ScanParams& p, const BwdIO& io,
+                                  hipStream_t st);
+template <int TY>
+hipError_t launch_scan_bwd_fast_walk(int S, int NPL, int gk, const ScanParams& p, const BwdIO& io,
+                                     hipStream_t st);
+// The tile-walking launches of the general instantiation.
+hipError_t launch_scan_bwd_walk(int S, int NPL, int gk, const ScanParams& p, const BwdIO& io,
+                                hipStream_t st);
+
+template <int S, int NPL, class GK, bool FAST, bool MULTI, int TY>
+hipError_t launch_bwd_kernel(const ScanParams& p, const BwdIO& io, hipStream_t st) {
+  dim3 grid((unsigned)((int64_t)io.ntg * io.nbg));
+  hipLaunchKernelGGL((scan_bwd_kernel<S, NPL, GK, FAST, MULTI, TY>), grid, dim3(kThreads), 0, st, p,
+                     io);
+  return hipGetLastError();
+}
 
 }  // namespace rp
