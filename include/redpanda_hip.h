@@ -28,7 +28,7 @@
 extern "C" {
 #endif
 
-#define RP_ABI_VERSION 13
+#define RP_ABI_VERSION 14
 
 /* element type codes of the streamed scan inputs (delta, u, Bc, Cc); each
  * tensor carries its own code, as autocast hands over mixed dtypes */
@@ -447,6 +447,55 @@ int rp_step(const rp_step_args* a, void* stream);
  * dominate (a Mamba.step ply at MARS's batch sizes).
  */
 int rp_step_bcnorm(const rp_step_args* a, const rp_bcnorm_args* bn, void* stream);
+
+/*
+ * One layer of the inference step in fp32, whole: the pre-norm, the
+ * projections, the step and the residual add of Mamba.step's loop
+ * (engine/mamba.py:440-498 and :592-597), as five launches from one call:
+ *   in_proj of norm(x) (SiLU on its first D outputs), x_proj, dt_proj,
+ *   rp_step_bcnorm (gated by z), x_out = x + out_proj.
+ * For small batches, where a layer is launches and latency: x is (R,
+ * d_model) with 16-byte aligned rows, every weight contiguous fp32 and
+ * 16-byte aligned, d_model, D and dt_rank multiples of 4.  in_w (2 D,
+ * d_model), xp_w (dt_rank + 2 N P, D), dtp_w (D, dt_rank), out_w (d_model,
+ * D); biases may be NULL.  State arguments as in rp_step_args; x_out (R,
+ * d_model) contiguous and not overlapping x.  work: rp_layer_step_work_bytes,
+ * 256-byte aligned.
+ */
+typedef struct rp_layer_step_args {
+  int64_t R, d_model, D, N, NR, NT, P, dt_rank;
+  const float* x;
+  int64_t x_sr;
+  const float* norm_w;
+  const float* in_w;
+  const float* in_b;
+  const float* xp_w;
+  const float* xp_b;
+  const float* dtp_w;
+  const float* dtp_b;
+  const float* out_w;
+  const float* out_b;
+  const float* bn_wB; /* (N P,) BCNorm weights, or NULL without BCNorm */
+  const float* bn_wC;
+  const float* A_real;
+  const float* A_imag;
+  const float* track;
+  const float* Dskip;
+  const float* h_in;
+  const float* beta_in;
+  float* h_out;
+  float* beta_out;
+  float* x_out;
+  void* work;
+  int64_t work_bytes;
+  float norm_eps, bn_eps;
+  int32_t broadcast_state, beta_rank1;
+} rp_layer_step_args;
+
+int rp_layer_step_check(const rp_layer_step_args* a);
+/* Bytes of work, or a negative status. */
+int64_t rp_layer_step_work_bytes(const rp_layer_step_args* a);
+int rp_layer_step(const rp_layer_step_args* a, void* stream);
 
 #ifdef __cplusplus
 }

@@ -13,7 +13,7 @@ import torch
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libredpanda_hip.so")
 
-ABI_VERSION = 13
+ABI_VERSION = 14
 RP_F32, RP_BF16, RP_F16 = 0, 1, 2
 DTYPE_CODES = {torch.float32: RP_F32, torch.bfloat16: RP_BF16, torch.float16: RP_F16}
 MAX_STATE = 128
@@ -103,6 +103,22 @@ class RmsNormArgs(ctypes.Structure):
     ]
 
 
+class LayerStepArgs(ctypes.Structure):
+    _fields_ = [
+        ("R", _i64), ("d_model", _i64), ("D", _i64), ("N", _i64), ("NR", _i64), ("NT", _i64),
+        ("P", _i64), ("dt_rank", _i64),
+        ("x", _vp), ("x_sr", _i64), ("norm_w", _vp),
+        ("in_w", _vp), ("in_b", _vp), ("xp_w", _vp), ("xp_b", _vp),
+        ("dtp_w", _vp), ("dtp_b", _vp), ("out_w", _vp), ("out_b", _vp),
+        ("bn_wB", _vp), ("bn_wC", _vp),
+        ("A_real", _vp), ("A_imag", _vp), ("track", _vp), ("Dskip", _vp),
+        ("h_in", _vp), ("beta_in", _vp), ("h_out", _vp), ("beta_out", _vp),
+        ("x_out", _vp), ("work", _vp), ("work_bytes", _i64),
+        ("norm_eps", ctypes.c_float), ("bn_eps", ctypes.c_float),
+        ("broadcast_state", _i32), ("beta_rank1", _i32),
+    ]
+
+
 class PlyTopkArgs(ctypes.Structure):
     _fields_ = [
         ("R", _i64), ("V", _i64), ("k", _i32), ("dtype_logits", _i32),
@@ -136,6 +152,9 @@ SIGNATURES = {
     "rp_bcnorm_fwd": (ctypes.c_int, [ctypes.POINTER(BcNormArgs), _vp]),
     "rp_bcnorm_bwd": (ctypes.c_int, [ctypes.POINTER(BcNormArgs), ctypes.POINTER(BcNormGrad), _vp]),
     "rp_step_bcnorm": (ctypes.c_int, [ctypes.POINTER(StepArgs), ctypes.POINTER(BcNormArgs), _vp]),
+    "rp_layer_step_check": (ctypes.c_int, [ctypes.POINTER(LayerStepArgs)]),
+    "rp_layer_step_work_bytes": (_i64, [ctypes.POINTER(LayerStepArgs)]),
+    "rp_layer_step": (ctypes.c_int, [ctypes.POINTER(LayerStepArgs), _vp]),
     "rp_rmsnorm_check": (ctypes.c_int, [ctypes.POINTER(RmsNormArgs)]),
     "rp_rmsnorm_fwd": (ctypes.c_int, [ctypes.POINTER(RmsNormArgs), _vp]),
     "rp_softplus": (ctypes.c_int, [_vp, _vp, _i64, _vp]),

@@ -675,6 +675,173 @@ int rp_step_bcnorm(const rp_step_args* a, const rp_bcnorm_args* bn, void* stream
 
 }  // extern "C"
 
+// ── one layer of the inference step ──
+
+namespace {
+
+// Float offsets of the layer step's intermediates in its workspace.
+struct LayerStepPlan {
+  int64_t xz, proj, dt, Bc, Cc, y, floats;
+  int64_t proj_w, proj_sr;  // x_proj outputs per row, and the row stride
+};
+
+LayerStepPlan layer_step_plan(const rp_layer_step_args* a) {
+  LayerStepPlan l{};
+  l.proj_w = a->dt_rank + 2 * a->N * a->P;
+  l.proj_sr = round_up(l.proj_w, 4);  // dt_proj reads 16-byte vectors of its rows
+  int64_t at = 0;
+  auto take = [&](int64_t n) {
+    const int64_t o = at;
+    at += round_up(n, 64);  // 256-byte blocks
+    return o;
+  };
+  l.xz = take(a->R * 2 * a->D);
+  l.proj = take(a->R * l.proj_sr);
+  l.dt = take(a->R * a->D);
+  l.Bc = take(a->R * a->N);
+  l.Cc = take(a->R * a->N);
+  l.y = take(a->R * a->D);
+  l.floats = at;
+  return l;
+}
+
+// The layer step's own arguments (those of the step and of BCNorm are checked
+// by rp_step_bcnorm, before anything is launched).
+int layer_step_check(const rp_layer_step_args* a) {
+  if (a == nullptr) return fail(RP_ERR_INVALID, "layer step args: NULL");
+  if (a->R < 0 || a->d_model < 1 || a->D < 1 || a->N < 1 || a->P < 1 || a->dt_rank < 1)
+    return fail(RP_ERR_INVALID, "layer step args: bad size");
+  if (a->d_model % 4 || a->D % 4 || a->dt_rank % 4)
+    return fail(RP_ERR_UNSUPPORTED,
+                "layer step args: d_model, D and dt_rank must be multiples of 4");
+  if (a->R > (1 << 20) || a->d_model > (1 << 20) || a->D > (1 << 20) || a->dt_rank > (1 << 20) ||
+      a->N > RP_MAX_STATE || a->P > (1 << 10))
+    return fail(RP_ERR_UNSUPPORTED, "layer step args: size beyond the limits");
+  return RP_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int64_t rp_layer_step_work_bytes(const rp_layer_step_args* a) {
+  const int st = layer_step_check(a);
+  return st != RP_OK ? st : layer_step_plan(a).floats * 4;
+}
+
+int rp_layer_step_check(const rp_layer_step_args* a) {
+  const int st = layer_step_check(a);
+  if (st != RP_OK) return st;
+  if (a->R == 0) return RP_OK;
+  // rows read as 16-byte vectors
+  const void* vec[] = {a->x, a->norm_w, a->in_w, a->xp_w, a->dtp_w, a->out_w};
+  for (const void* q : vec)
+    if (!q || !aligned(q, 16)) return fail(RP_ERR_INVALID, "layer step args: NULL or misaligned operand");
+  if (a->x_sr < a->d_model || a->x_sr % 4)
+    return fail(RP_ERR_INVALID, "layer step args: x row stride");
+  const void* other[] = {a->in_b, a->xp_b, a->dtp_b, a->out_b, a->x_out, a->bn_wB, a->bn_wC};
+  for (const void* q : other)
+    if (q && !aligned(q, 4)) return fail(RP_ERR_INVALID, "layer step args: misaligned pointer");
+  if (!a->x_out) return fail(RP_ERR_INVALID, "layer step args: NULL x_out");
+  if ((a->bn_wB == nullptr) != (a->bn_wC == nullptr))
+    return fail(RP_ERR_INVALID, "layer step args: the BCNorm weights go together");
+  if (!(a->norm_eps >= 0.f)) return fail(RP_ERR_INVALID, "layer step args: norm_eps must be >= 0");
+  if (overlaps(a->x_out, a->R * a->d_model * 4, a->x, ((a->R - 1) * a->x_sr + a->d_model) * 4))
+    return fail(RP_ERR_INVALID, "layer step args: x_out overlaps x");
+  if (!a->work || !aligned(a->work, 256) || a->work_bytes < layer_step_plan(a).floats * 4)
+    return fail(RP_ERR_WORKSPACE, "layer step: workspace missing, misaligned or too small");
+  return RP_OK;
+}
+
+int rp_layer_step(const rp_layer_step_args* a, void* stream) {
+  int st = rp_layer_step_check(a);
+  if (st != RP_OK) return st;
+  if (a->R == 0) return RP_OK;
+  const LayerStepPlan l = layer_step_plan(a);
+  float* w = static_cast<float*>(a->work);
+  rp_step_args s{};
+  s.R = a->R;
+  s.D = a->D;
+  s.N = a->N;
+  s.NR = a->NR;
+  s.NT = a->NT;
+  s.delta = w + l.dt;
+  s.delta_sr = a->D;
+  s.u = w + l.xz;
+  s.u_sr = 2 * a->D;
+  s.Bc = w + l.Bc;
+  s.Bc_sr = a->N;
+  s.Cc = w + l.Cc;
+  s.Cc_sr = a->N;
+  s.h_in = a->h_in;
+  s.beta_in = a->beta_in;
+  s.A_real = a->A_real;
+  s.A_imag = a->A_imag;
+  s.track = a->track;
+  s.Dskip = a->Dskip;
+  s.h_out = a->h_out;
+  s.beta_out = a->beta_out;
+  s.y = w + l.y;
+  s.broadcast_state = a->broadcast_state;
+  s.delta_softplus = 1;
+  s.beta_rank1 = a->beta_rank1;
+  s.z = w + l.xz + a->D;
+  s.z_sr = 2 * a->D;
+  s.dtype_z = RP_F32;
+  rp_bcnorm_args bn{};
+  bn.T = a->R;
+  bn.N = a->N;
+  bn.P = a->P;
+  bn.dtype_x = RP_F32;
+  bn.normalize = a->bn_wB != nullptr;
+  bn.eps = a->bn_eps;
+  bn.B_raw = w + l.proj + a->dt_rank;
+  bn.B_sr = l.proj_sr;
+  bn.C_raw = w + l.proj + a->dt_rank + a->N * a->P;
+  bn.C_sr = l.proj_sr;
+  bn.wB = a->bn_wB;
+  bn.wC = a->bn_wC;
+  bn.Bc = w + l.Bc;
+  bn.Cc = w + l.Cc;
+  // the step's arguments are checked before the first launch
+  st = rp_step_check(&s);
+  if (st == RP_OK) st = rp_bcnorm_check(&bn);
+  if (st != RP_OK) return st;
+  auto linear = [&](int mode, const float* x, int64_t xsr, int64_t K, const float* wt,
+                    const float* bias, int64_t N, float* out, int64_t osr) -> int {
+    rp::LinearParams p{};
+    p.R = (int)a->R;
+    p.K = (int)K;
+    p.N = (int)N;
+    p.x = x;
+    p.xsr = xsr;
+    p.w = wt;
+    p.bias = bias;
+    p.norm_w = a->norm_w;
+    p.eps = a->norm_eps;
+    p.nsilu = (int)a->D;
+    p.add = a->x;
+    p.asr = a->x_sr;
+    p.out = out;
+    p.osr = osr;
+    const hipError_t e = rp::launch_linear(p, mode, (hipStream_t)stream);
+    return e != hipSuccess ? fail_hip(e, "linear launch") : RP_OK;
+  };
+  st = linear(rp::kLinNorm | rp::kLinSilu, a->x, a->x_sr, a->d_model, a->in_w, a->in_b, 2 * a->D,
+              w + l.xz, 2 * a->D);
+  if (st == RP_OK) st = linear(0, w + l.xz, 2 * a->D, a->D, a->xp_w, a->xp_b, l.proj_w, w + l.proj,
+                              l.proj_sr);
+  if (st == RP_OK)
+    st = linear(0, w + l.proj, l.proj_sr, a->dt_rank, a->dtp_w, a->dtp_b, a->D, w + l.dt, a->D);
+  if (st == RP_OK) st = rp_step_bcnorm(&s, &bn, stream);
+  if (st == RP_OK)
+    st = linear(rp::kLinAdd, w + l.y, a->D, a->D, a->out_w, a->out_b, a->d_model, a->x_out,
+                a->d_model);
+  return st;
+}
+
+}  // extern "C"
+
 // ── mixer output gate ──
 
 namespace {

@@ -175,6 +175,30 @@ constexpr int kBcNormWorkgroups = 1024;
 hipError_t launch_bcnorm_fwd(const BcNormParams& p, hipStream_t st);
 hipError_t launch_bcnorm_bwd(const BcNormParams& p, const BcNormGrad& g, hipStream_t st);
 
+// Small-batch fp32 linear layer out = x W^T (+ bias), rows of x and out
+// (linear.hip).
+constexpr int kLinWaves = 16;  // waves per workgroup, splitting K
+enum LinMode {
+  kLinNorm = 1,  // x RMS-normalised (norm_w, eps) on the way in
+  kLinSilu = 2,  // SiLU on the first nsilu outputs
+  kLinAdd = 4,   // out = add + x W^T
+};
+struct LinearParams {
+  int R, K, N;
+  const float* x;       // (R, K), row stride xsr; 16-byte aligned rows
+  int64_t xsr;
+  const float* w;       // (N, K) contiguous, K a multiple of 4, 16-byte aligned
+  const float* bias;    // (N,) or null
+  const float* norm_w;  // (K,), 16-byte aligned
+  float eps;
+  int nsilu;
+  const float* add;     // (R, N), row stride asr
+  int64_t asr;
+  float* out;           // (R, N), row stride osr
+  int64_t osr;
+};
+hipError_t launch_linear(const LinearParams& p, int mode, hipStream_t st);
+
 // Residual add + RMSNorm of rows (forward only).
 struct RmsNormParams {
   int64_t rows;

@@ -1,0 +1,118 @@
+"""One Mamba-3 layer of the inference step as a single library call.
+
+`hip_layer_step` is the body of Mamba.step's pre-norm loop for one layer
+(engine/mamba.py:592-597 around Mamba3Block.step, :440-498): x + out_proj of
+the gated step of norm(x), with the norm, SiLU and residual add folded into
+small-batch fp32 projections (rp_layer_step: five launches where the separate
+ops take seven, and one call from Python where they take eight).  Inference
+only.
+"""
+
+import ctypes
+
+import torch
+import torch.nn as nn
+from torch.nn.modules import module as _nn_module
+
+from redpanda_amd import _lib
+from redpanda_amd.step import _state_pair
+
+# Beyond this the separate launches, whose GEMMs then run at their own rate, were
+# not measured against it: at 8 layers of d_model 512, 12 / 64 / 256 rows, an
+# eager ply takes 0.50 / 0.49 / 0.58 ms against 1.32 / 1.32 / 1.35, a replayed
+# one 0.27 / 0.30 / 0.57 against 0.40 / 0.44 / 0.60.
+MAX_ROWS = 256
+
+
+def _plain_linear(m, out_features, in_features):
+    """A Linear of this shape that computes just that: no subclass,
+    parametrization or hook that a direct use of its weight would pass by."""
+    return (type(m) is nn.Linear and not m._forward_hooks and not m._forward_pre_hooks and
+            m.weight.shape == (out_features, in_features))
+
+
+def usable(model, x):
+    """Whether Mamba.step's inference loop may take hip_layer_step for the
+    rows x (R, d_model) fp32: a small batch, plain fp32 projections of the
+    configured shapes on x's device, contiguous and 16-byte aligned."""
+    cfg = model.config
+    d, D, r = cfg.d_model, cfg.d_inner, cfg.dt_rank
+    if x.shape[0] > MAX_ROWS or x.shape[0] == 0 or x.shape[1] != d or d % 4 or D % 4 or r % 4:
+        return False
+    if cfg.mimo_p > 8 or torch.is_autocast_enabled("cuda"):
+        return False
+    if _nn_module._global_forward_hooks or _nn_module._global_forward_pre_hooks:
+        return False
+    np2 = 2 * cfg.d_state * cfg.mimo_p
+    dev = x.device
+    for layer in model.layers:
+        mx = layer["mixer"]
+        if not (_plain_linear(mx.in_proj, 2 * D, d) and _plain_linear(mx.x_proj, r + np2, D) and
+                _plain_linear(mx.dt_proj, D, r) and _plain_linear(mx.out_proj, d, D)):
+            return False
+        ws = [mx.in_proj.weight, mx.x_proj.weight, mx.dt_proj.weight, mx.out_proj.weight,
+              layer["norm"].weight, mx.D]
+        for lin in (mx.in_proj, mx.x_proj, mx.dt_proj, mx.out_proj):
+            if lin.bias is not None:
+                ws.append(lin.bias)
+        if cfg.use_bcnorm:
+            ws += (mx.b_norm.weight, mx.c_norm.weight)
+        bits = 0
+        for w in ws:
+            if w.dtype is not torch.float32 or w.device != dev or not w.is_contiguous():
+                return False
+            bits |= w.data_ptr()
+        if bits & 15:
+            return False
+    return True
+
+
+def hip_layer_step(x, layer, state, compact=False, out=None):
+    """(x + layer(x), (h, beta)) for rows x (R, d_model) fp32 that `usable`
+    accepted; state, compact and out as in Mamba3Block.step."""
+    lib = _lib.load()
+    mx = layer["mixer"]
+    cfg = mx.config
+    R, D, N = x.shape[0], cfg.d_inner, cfg.d_state
+    dev = x.device
+    if x.stride(-1) != 1 or x.stride(0) % 4 or x.data_ptr() & 15:
+        x = x.contiguous()
+    Ar, Ai, Tk = mx._gates(False)
+    a = _lib.LayerStepArgs()
+    a.R, a.d_model, a.D, a.N = R, cfg.d_model, D, N
+    a.NR, a.NT, a.P, a.dt_rank = cfg.n_rot_state, cfg.n_track_state, cfg.mimo_p, cfg.dt_rank
+    h_in = beta_in = None
+    rank1 = bool(compact)
+    if state is not None:
+        h_in, beta_in, broadcast, rank1 = _state_pair(state[0], state[1], R, D, N)
+        a.h_in, a.beta_in, a.broadcast_state = h_in.data_ptr(), beta_in.data_ptr(), broadcast
+    bshape = (R, D + N) if rank1 else (R, D, N)
+    f32 = dict(dtype=torch.float32, device=dev)
+    if out is None:
+        h_out, beta_out = torch.empty((R, D, N), **f32), torch.empty(bshape, **f32)
+    else:
+        h_out, beta_out = out
+        for name, t, shp in (("h", h_out, (R, D, N)), ("beta", beta_out, bshape)):
+            if (t.shape != shp or t.dtype != torch.float32 or t.device != dev or
+                    not t.is_contiguous()):
+                raise ValueError(f"step: out {name} must be a contiguous fp32 {shp} tensor on {dev}")
+    x_out = torch.empty((R, cfg.d_model), **f32)
+    norm = layer["norm"]
+    a.x, a.x_sr, a.norm_w, a.norm_eps = x.data_ptr(), x.stride(0), norm.weight.data_ptr(), norm.eps
+    for pre, lin in (("in", mx.in_proj), ("xp", mx.x_proj), ("dtp", mx.dt_proj), ("out", mx.out_proj)):
+        setattr(a, pre + "_w", lin.weight.data_ptr())
+        if lin.bias is not None:
+            setattr(a, pre + "_b", lin.bias.data_ptr())
+    if cfg.use_bcnorm:
+        a.bn_wB, a.bn_wC, a.bn_eps = (mx.b_norm.weight.data_ptr(), mx.c_norm.weight.data_ptr(),
+                                      mx.b_norm.eps)
+    a.A_real, a.A_imag, a.track = _lib.ptr(Ar), _lib.ptr(Ai), _lib.ptr(Tk)
+    a.Dskip = mx.D.data_ptr()
+    a.h_out, a.beta_out, a.x_out = h_out.data_ptr(), beta_out.data_ptr(), x_out.data_ptr()
+    a.beta_rank1 = 1 if rank1 else 0
+    nbytes = lib.rp_layer_step_work_bytes(ctypes.byref(a))
+    _lib.check(0 if nbytes >= 0 else -1, lib)
+    work = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    a.work, a.work_bytes = work.data_ptr(), nbytes
+    _lib.check(lib.rp_layer_step(ctypes.byref(a), _lib.stream_of(dev)), lib)
+    return x_out, (h_out, beta_out)

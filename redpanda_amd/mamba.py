@@ -33,6 +33,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 import torch.utils.checkpoint
 
+from redpanda_amd import layer_step
 from redpanda_amd.bcnorm import hip_bcnorm_psum
 from redpanda_amd.mixer import hip_mixer_out
 from redpanda_amd.norm import hip_add_rmsnorm
@@ -408,6 +409,15 @@ class Mamba(nn.Module):
             x.requires_grad or any(p.requires_grad for p in self.parameters()) or
             any(t.requires_grad for st in cache if st is not None for t in st))
         if not record and x.dtype == torch.float32 and x.dim() == 2 and len(self.layers) > 0:
+            if layer_step.usable(self, x):
+                # a small batch of plain fp32 layers: one library call each
+                for i, layer in enumerate(self.layers):
+                    x, st = layer_step.hip_layer_step(x, layer, cache[i], compact=compact,
+                                                      out=None if out_cache is None else out_cache[i])
+                    new_cache.append(st)
+                if apply_final_norm:
+                    _, x = hip_add_rmsnorm(x, None, self.norm_f.weight, self.norm_f.eps)
+                return x, new_cache
             # inference: each layer's residual add and the next RMSNorm (the
             # next layer's, or norm_f) in one fused pass
             _, xn = hip_add_rmsnorm(x, None, self.layers[0]["norm"].weight,
