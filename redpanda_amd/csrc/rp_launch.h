@@ -285,6 +285,21 @@ inline int gate_code_all(bool has_imag, int64_t NR, int64_t N, int S, int NPL) {
 
 hipError_t launch_scan_fwd(int S, int NPL, int gk, const ScanParams& p, const FwdOut& o,
                            hipStream_t st);
+// The storage types of a scan forward instantiation (FwdTypes in
+// scan_fwd_kernel.h).
+enum FwdTypeCode {
+  kFwdAny = 0,        // any mix, read at run time
+  kFwdF32 = 1,        // all fp32
+  kFwdBf16 = 2,       // all bf16
+  kFwdF16 = 3,        // all fp16
+  kFwdModelBf16 = 4,  // softplus on load, delta and u in bf16, B and C in fp32
+  kFwdModelF16 = 5,   // the same with fp16
+  kFwdF32Sp = 6,      // softplus on load, all fp32
+  kFwdMixBf16 = 7,    // u in bf16, the rest fp32 (the reference's autocast call)
+};
+template <int TY>
+hipError_t launch_scan_fwd_ty(int S, int NPL, int gk, const ScanParams& p, const FwdOut& o,
+                              hipStream_t st);
 hipError_t launch_scan_bwd(int S, int NPL, int gk, const ScanParams& p, const BwdIO& io,
                            hipStream_t st);
 hipError_t launch_bwd_finalize(const ScanParams& p, const BwdIO& io, float* d_Bc, float* d_Cc,

@@ -1,0 +1,6 @@
+// The scan forward's instantiations (scan_fwd_kernel.h): the model's launches under bf16 autocast.
+#include "scan_fwd_kernel.h"
+
+namespace rp {
+template hipError_t launch_scan_fwd_ty<kFwdModelBf16>(int, int, int, const ScanParams&, const FwdOut&, hipStream_t);
+}
