@@ -628,10 +628,21 @@ int step_impl(const rp_step_args* a, const rp_bcnorm_args* bn, void* stream) {
       ri = (a->R * (int64_t)p.ctiles) / 512;
       if (ri < 1) ri = 1;
       if (ri > ri_max) ri = ri_max;
+      // 16 slices in 4 threads per channel and no pad states (d_state 48, 64),
+      // full beta: one rollout per workgroup up to 12288 workgroups, whose
+      // kernel loads the gates as vectors and its state ahead of the prologue
+      // (d_state 64, D 1024: 18 / 62 / 115 us at 64 / 256 / 512 rollouts, 22 /
+      // 67 / 124 with several; at 1024 rollouts 219 against 213, and with pad
+      // states 67 against 55 at 256)
+      if (S == 16 && rp::step_tile_split(S, NPL) == 4 && !a->beta_rank1 && !a->broadcast_state &&
+          a->delta_softplus && a->N == S * NPL && a->R * (int64_t)p.ctiles <= 12288)
+        ri = 1;
     }
     if (ri > rp::step_tile_ri_max(S, NPL, a->beta_rank1 != 0))
       return fail(RP_ERR_UNSUPPORTED, "step: rollouts per workgroup");
     p.ri = (int)ri;
+    p.gate_vec = a->NR % 4 == 0 && a->NT % 4 == 0 && aligned(p.Ar, 16) && aligned(p.Ai, 16) &&
+                 aligned(p.Tk, 16);
     p.rgroups = (int)((a->R + ri - 1) / ri);
     if ((int64_t)p.ctiles * p.rgroups > kI32Max)
       return fail(RP_ERR_UNSUPPORTED, "step: grid too large");

@@ -93,6 +93,7 @@ struct StepParams {
   int ctiles;   // tile kernel: channel tiles of kStepTile / step_tile_split(S, NPL)
   int ri;       // tile kernel: rollouts per workgroup
   int rgroups;  // tile kernel: ceil(R / ri)
+  int gate_vec; // tile kernel: NR, NT multiples of 4, gate arrays 16-byte aligned
   // tile kernel, one rollout per workgroup: the B / C rows computed in the
   // prologue from the raw projections (BCNorm + p-sum) instead of read
   int bn_fused;
@@ -309,6 +310,8 @@ hipError_t launch_bwd_finalize(const ScanParams& p, const BwdIO& io, float* d_Bc
 // launch_step_tile_pad); otherwise the lane-layout kernel.  Bitwise the same.
 hipError_t launch_step(int S, int NPL, int gk, bool tile, const StepParams& p, hipStream_t st);
 hipError_t launch_step_tile_pad(int S, int NPL, int gk, const StepParams& p, hipStream_t st);
+hipError_t launch_step_tile_pad16(int S, int NPL, int gk, const StepParams& p, hipStream_t st);
+hipError_t launch_step_tile16(int S, int NPL, int gk, const StepParams& p, hipStream_t st);
 hipError_t launch_fill_zero(float* p, int64_t n, hipStream_t st);
 
 // Rollout-ply boundary (ply.hip).

@@ -125,9 +125,10 @@ hipError_t launch_fill_zero(float* p, int64_t n, hipStream_t st) {
 hipError_t launch_step(int S, int NPL, int gk, bool tile, const StepParams& p, hipStream_t st) {
   if (tile && p.N != S * NPL) return launch_step_tile_pad(S, NPL, gk, p, st);
   if (tile) {
+    if (S == 16) return launch_step_tile16(S, NPL, gk, p, st);
 #define RP_CASE(SS, NN) \
     if (S == SS && NN == NPL) return launch_step_tile<SS, NN, false>(gk, p, st);
-    RP_FOR_EACH_SHAPE(RP_CASE)
+    RP_FOR_EACH_SHAPE_4_8(RP_CASE)
 #undef RP_CASE
     return hipErrorInvalidValue;
   }

@@ -59,7 +59,12 @@ __device__ __forceinline__ void store_stream(float4* p, float4 v) {
 // and in the LDS block is N floats; the slots' states n >= N are pad states,
 // held as the lane-layout kernel and the scan hold them (zero state, zero
 // B / C, zero beta_prev), so that y's sum over the slices keeps its bits.
-template <int S, int NPL, class GK, bool FULLD, bool DSP, bool RANK1, bool SHARED, bool PAD>
+// ONE: one rollout per workgroup (p.ri == 1: small batches, where a launch is
+// latency).  Its state, dt, u and z are loaded ahead of the prologue, so that
+// their trip to memory overlaps the gate parameters' and the B / C rows'; with
+// several rollouts the registers that takes cost more than the first one gains.
+template <int S, int NPL, class GK, bool FULLD, bool DSP, bool RANK1, bool SHARED, bool PAD,
+          bool ONE>
 __global__ __launch_bounds__(kThreads) void step_tile_kernel(StepParams p) {
   static_assert(FULLD || !SHARED, "the shared-state instantiation is for whole tiles");
   constexpr int NP = S * NPL;
@@ -125,6 +130,33 @@ __global__ __launch_bounds__(kThreads) void step_tile_kernel(StepParams p) {
   const bool has_imag = p.Ai != nullptr;
   const int r_lo = rg * p.ri;
   const int nr = min(p.R, r_lo + p.ri) - r_lo;  // <= RIM (checked by the host)
+  // a rollout's block of the input state: its own, or the one shared state
+  // (ssr == 0)
+  auto load_block = [&](int64_t r, float4 (&hl)[NB], float4 (&bl)[NB]) {
+    const int64_t iblk = r * (p.ssr / 4) + (int64_t)c0 * NVM;
+    const float4* hi4 = reinterpret_cast<const float4*>(p.h_in) + iblk;
+    const float4* bi4 = reinterpret_cast<const float4*>(p.beta_in) + iblk;
+#pragma unroll
+    for (int m = 0; m < NB; ++m) {
+      const int k = tid + m * kThreads;
+      if ((FULLD && !PAD && WHOLE) || k < nvalid) {
+        hl[m] = SHARED ? hi4[k] : load_stream(hi4 + k);
+        if constexpr (!RANK1) bl[m] = SHARED ? bi4[k] : load_stream(bi4 + k);
+      }
+    }
+  };
+  // ONE: the rollout's inputs, ahead of the prologue's loads
+  float dt1 = 0.f, u1 = 0.f, z1 = 0.f, dtup1 = 0.f;
+  float4 h1[ONE ? NB : 1], b1[ONE ? NB : 1];
+  if constexpr (ONE) {
+    dt1 = p.delta[(int64_t)r_lo * p.dsr + cld];
+    u1 = p.u[(int64_t)r_lo * p.usr + cld];
+    if (p.z != nullptr) z1 = load_in(p.z, (int64_t)r_lo * p.zsr + cld, p.dt_z);
+    if (p.h_in != nullptr) {
+      if constexpr (RANK1) dtup1 = p.beta_in[(int64_t)r_lo * p.bssr + cld];
+      load_block(r_lo, h1, b1);
+    }
+  }
   // The prologue issues every load (B / C rows, gate parameters, D) before
   // it stores anything, so their latencies overlap.  The B / C rows of all
   // the workgroup's rollouts are staged once, pad states as zeros.
@@ -150,9 +182,38 @@ __global__ __launch_bounds__(kThreads) void step_tile_kernel(StepParams p) {
   auto st_n = [&](int i) { return (i / SS) * S + half * SS + i % SS; };
   // the thread's gate parameters stay in registers for all its rollouts
   GateRaw graw[NPT];
+  // VEC: with rows of 16-byte multiples the SS adjacent states of a slot are
+  // all rotational, all tracking or all padding, and load as one vector.  A
+  // wave's lanes read 64 different rows, so the scalar form's NPT loads (two
+  // per rotational state) keep the address unit busy for microseconds before
+  // the first state arrives: with ONE's early loads 8.3 -> 5.2 us at 1 rollout
+  // and 10.0 -> 6.8 at 64 (D 1024, 16 + 4 states), 262 -> 254 at 4096; rank-1
+  // rows 43 -> 33 at 777 and 149 -> 136 at 4096.  Not with 16 slices, the full
+  // beta and several rollouts per workgroup: there the scalar form stays (64
+  // states, 4096 rollouts: 780 us, 819 with vectors).
+  constexpr bool VEC = S != 16 || RANK1 || ONE;
+  if (VEC && p.gate_vec) {
 #pragma unroll
-  for (int i = 0; i < NPT; ++i)
-    graw[i] = gate_param_load(p.Ar, p.Ai, p.Tk, cld, st_n(i), N, p.NR, p.NT, true);
+    for (int v = 0; v < NVT; ++v) {
+      const int n = st_n(v * SS);
+      const bool rot = n < p.NR, trk = !rot && n < N;
+      const int64_t ir = rot ? (int64_t)cld * p.NR + n : 0;
+      const int64_t it = trk ? (int64_t)cld * p.NT + (n - p.NR) : 0;
+      V ar{}, ai{}, tk{};
+      if (v < GK::kTJ && p.NR > 0) {
+        ar = *reinterpret_cast<const V*>(p.Ar + ir);
+        if (has_imag) ai = *reinterpret_cast<const V*>(p.Ai + ir);
+      }
+      if (v >= GK::kRJ && p.NT > 0) tk = *reinterpret_cast<const V*>(p.Tk + it);
+#pragma unroll
+      for (int q = 0; q < SS; ++q)
+        graw[v * SS + q] = GateRaw{(&ar.x)[q], (&ai.x)[q], (&tk.x)[q]};
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < NPT; ++i)
+      graw[i] = gate_param_load(p.Ar, p.Ai, p.Tk, cld, st_n(i), N, p.NR, p.NT, true);
+  }
   const float dsk = p.Dskip[cld];
   if (p.bn_fused) {
     // the B and C rows of the workgroup's rollout from the raw projections:
@@ -197,28 +258,15 @@ __global__ __launch_bounds__(kThreads) void step_tile_kernel(StepParams p) {
   for (int rr = 0; rr < nr; ++rr) {
     const int64_t r = r_lo + rr;
     const int64_t blk = (r * p.D + c0) * NVM;  // float4 offset of the output block
-    float dt = p.delta[r * p.dsr + cld];
+    float dt = ONE ? dt1 : p.delta[r * p.dsr + cld];
     if constexpr (DSP) dt = softplus_of(dt);
-    const float uu = p.u[r * p.usr + cld];
+    const float uu = ONE ? u1 : p.u[r * p.usr + cld];
     // the gate branch, when y leaves gated
-    const float zz = p.z != nullptr ? load_in(p.z, r * p.zsr + cld, p.dt_z) : 0.f;
+    float zz = z1;
+    if constexpr (!ONE) zz = p.z != nullptr ? load_in(p.z, r * p.zsr + cld, p.dt_z) : 0.f;
     // rank-1: the channel's (dt*u)_prev, halved as the scan halves dt*u
     float hdp = 0.f;
-    if (p.h_in != nullptr) {
-      if constexpr (RANK1) hdp = 0.5f * p.beta_in[r * p.bssr + cld];
-      // input block: the rollout's own, or the one shared state (ssr == 0)
-      const int64_t iblk = r * (p.ssr / 4) + (int64_t)c0 * NVM;
-      const float4* hi4 = reinterpret_cast<const float4*>(p.h_in) + iblk;
-      const float4* bi4 = reinterpret_cast<const float4*>(p.beta_in) + iblk;
-      float4 hl[NB], bl[NB];
-#pragma unroll
-      for (int m = 0; m < NB; ++m) {
-        const int k = tid + m * kThreads;
-        if ((FULLD && !PAD && WHOLE) || k < nvalid) {
-          hl[m] = SHARED ? hi4[k] : load_stream(hi4 + k);
-          if constexpr (!RANK1) bl[m] = SHARED ? bi4[k] : load_stream(bi4 + k);
-        }
-      }
+    auto store_block = [&](const float4 (&hl)[NB], const float4 (&bl)[NB]) {
 #pragma unroll
       for (int m = 0; m < NB; ++m) {
         const int k = tid + m * kThreads;
@@ -226,6 +274,17 @@ __global__ __launch_bounds__(kThreads) void step_tile_kernel(StepParams p) {
           sH[k] = hl[m];
           if constexpr (!RANK1) sBt[k] = bl[m];
         }
+      }
+    };
+    if (p.h_in != nullptr) {
+      if constexpr (ONE) {
+        if constexpr (RANK1) hdp = 0.5f * dtup1;
+        store_block(h1, b1);
+      } else {
+        if constexpr (RANK1) hdp = 0.5f * p.beta_in[r * p.bssr + cld];
+        float4 hl[NB], bl[NB];
+        load_block(r, hl, bl);
+        store_block(hl, bl);
       }
     } else {
 #pragma unroll
@@ -331,14 +390,22 @@ template <int S, int NPL, class GK, bool DSP, bool RANK1, bool PAD>
 hipError_t launch_step_tile_d(const StepParams& p, hipStream_t st) {
   dim3 grid((unsigned)((int64_t)p.ctiles * p.rgroups));
   const int tch = kThreads / step_tile_split(S, NPL);
+  // (the model's steps are the DSP ones)
+  const bool one = DSP && p.ri == 1;
   if (p.D % tch == 0 && p.ssr == 0)
-    hipLaunchKernelGGL((step_tile_kernel<S, NPL, GK, true, DSP, RANK1, true, PAD>), grid,
+    hipLaunchKernelGGL((step_tile_kernel<S, NPL, GK, true, DSP, RANK1, true, PAD, false>), grid,
+                       dim3(kThreads), 0, st, p);
+  else if (p.D % tch == 0 && one)
+    hipLaunchKernelGGL((step_tile_kernel<S, NPL, GK, true, DSP, RANK1, false, PAD, DSP>), grid,
                        dim3(kThreads), 0, st, p);
   else if (p.D % tch == 0)
-    hipLaunchKernelGGL((step_tile_kernel<S, NPL, GK, true, DSP, RANK1, false, PAD>), grid,
+    hipLaunchKernelGGL((step_tile_kernel<S, NPL, GK, true, DSP, RANK1, false, PAD, false>), grid,
+                       dim3(kThreads), 0, st, p);
+  else if (one)
+    hipLaunchKernelGGL((step_tile_kernel<S, NPL, GK, false, DSP, RANK1, false, PAD, DSP>), grid,
                        dim3(kThreads), 0, st, p);
   else
-    hipLaunchKernelGGL((step_tile_kernel<S, NPL, GK, false, DSP, RANK1, false, PAD>), grid,
+    hipLaunchKernelGGL((step_tile_kernel<S, NPL, GK, false, DSP, RANK1, false, PAD, false>), grid,
                        dim3(kThreads), 0, st, p);
   return hipGetLastError();
 }
