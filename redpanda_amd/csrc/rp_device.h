@@ -241,9 +241,10 @@ __device__ __forceinline__ float ffma(float a, float b, float c) { return __buil
 // exp2 on the transcendental unit (v_exp_f32).
 __device__ __forceinline__ float exp2_hw(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// The gate table copied into LDS once per workgroup (read after the
-// workgroup's next barrier): the sign-folded records (m, b (-sin a)) of the
-// kTab table angles 2 pi k / kTab (the backward: fill_sincos_fine).
+// The gate tables copied into LDS once per workgroup (read after the
+// workgroup's next barrier): the sign-folded records (m, b (-sin a))
+// (forward and step) or (m, b sin) (backward) of the kTab table angles
+// 2 pi k / kTab.
 __device__ __forceinline__ void fill_cos_lin(float2* ctab, int tid) {
   for (int k = tid; k < kTab; k += kThreads) ctab[k] = kCosLin[k];
 }
@@ -254,6 +255,10 @@ __device__ __forceinline__ void fill_cos_lin(float4* ctab, int tid) {
     const float2 rec = kCosLin[k], pc = cos_lin_coefs(rec);
     ctab[k] = make_float4(rec.x, rec.y, pc.x, pc.y);
   }
+}
+
+__device__ __forceinline__ void fill_sincos_pairs(float2* cstab, int tid) {
+  for (int k = tid; k < kTab; k += kThreads) cstab[k] = kSinCos[k];
 }
 
 // Per-state gate parameters held in registers: pah = fl(A_real log2(e)) and
@@ -296,6 +301,7 @@ __device__ __forceinline__ void gate_param_finish(int n, int N, int NR, bool val
   wh = rot ? wr : 0.f;
 }
 
+constexpr float kRadPerStep = 0.02454369328916073f;  // 2 pi / 256: radians per table step
 constexpr float kRint = 12582912.f;  // 1.5 * 2^23: x + kRint rounds x to an integer
 // With a = 2 pi / 256 and |r| <= 1/2:  cos(a r) - 1 = kC2 r^2  (truncation
 // < 9.5e-10),  sin(a r) = r (kS1 + kS3 r^2)  (truncation < 2.4e-12)
@@ -336,9 +342,10 @@ __device__ __forceinline__ int angle_split(float dt, float wh, float& r) {
 //   * the forward and the step: w = cos/b - 1 as the cubic in r from the
 //     index's record (m, b (-s a)) (one 8-byte table read; the two higher
 //     coefficients one operation each, then three FMAs);
-//   * the backward: w as the quadratic in r, and -a b sin as its derivative,
-//     from a finer table's record (one 8-byte read; fill_sincos_fine).  Its
-//     gate is the forward's to within an ulp.
+//   * the backward: w and also b sin from the index's record (m, b s) (one
+//     8-byte read; the two expansions share r^2, cos(a r) - 1 and sin(a r)).
+//     Its gate is the forward's to within an ulp (the same expansion,
+//     rounded differently).
 // Both return the gate as (b e)(1 + w), b e = e with the sign bit of m.
 // R: the forward's table record, (m, b (-s a)) as float2, or as float4 with
 // the expansion's two record-only coefficients (p3, p2) appended (taken at
@@ -353,7 +360,7 @@ struct GatePart {
 struct GatePartCS {
   float e;
   float r;
-  float2 cs;  // (m, b (-s a)) of the table angle, a = 2 pi / kTabB
+  float2 cs;  // (m, b s) of the table angle
 };
 
 // e (>= 0) with the sign bit of m: b e for a sign-folded record.
@@ -397,63 +404,8 @@ __device__ __forceinline__ float rot_gate_finish(const GatePart<R>& g, bool imag
   return ffma(be, w, be);
 }
 
-// The backward's table: kTabB angles, read with the remainder |r| <= 1/2 in
-// its own steps of a = 2 pi / kTabB, where the angle a r is below pi / 2048.
-// cos(a r) - 1 = kC2B r^2 and sin(a r) = a r are then accurate to 6e-10, so
-// the gate's expansion is a quadratic and the sine is its derivative: 9
-// operations for both, where the 256-entry table's cubics took 13: the
-// backward 2.65 -> 2.47 ms at the Eval-Mamba shape (with the (B, C) pairs and
-// unpadded row partials in LDS that make room for the table), 14.8 -> 13.5 ms
-// on the long sequence (B 64, L 2048, D 1024, N 72).  16 KB of LDS, which the
-// backward has (the forward needs its LDS for occupancy).
-constexpr int kTabB = 2048;
-constexpr float kC2B = -4.706194115204505e-06f;  // -a^2 / 2
-// sums of (-a sin) terms to sums of sin terms
-constexpr double kInvStepB = -325.94932345220167;  // -1 / a
-
-// Fills it from the 256-entry table: entry k lies r = off / 8 steps from the
-// nearest entry of kSinCos, off in [-4, 4), where cos / b - 1 and sin / b are
-// that entry's expansion (in float64, from its rounded record), the cosine's
-// sign b taken anew where it changes within the step.
-__device__ __forceinline__ void fill_sincos_fine(float2* tab, int tid) {
-  constexpr int kSub = kTabB / kTab;
-  static_assert(kSub == 8, "entries per step of the 256-entry table");
-  for (int k = tid; k < kTabB; k += kThreads) {
-    const int q = (k + kSub / 2) / kSub;
-    const double r = (double)(k - q * kSub) / kSub;
-    const float2 rec = kSinCos[q & (kTab - 1)];
-    const double am = fabsf(rec.x), sb = rec.y, r2 = r * r;
-    const double cm1 = r2 * (double)kC2;
-    const double sx = r * (r2 * (double)kS3 + (double)kS1);
-    double m = am - cm1 + am * cm1 + sb * sx;  // 1 - cos / b
-    double sn = sb + sb * cm1 + sx - am * sx;  // sin / b
-    double sg = signbit(rec.x) ? -1.0 : 1.0;
-    if (m > 1.0) {
-      m = 2.0 - m;
-      sn = -sn;
-      sg = -sg;
-    }
-    tab[k] = make_float2((float)(sg * m), (float)(sn * (1.0 / kInvStepB)));
-  }
-}
-
-// The angle in the table's steps split into an integer, whose low bits are
-// the entry's index, and a remainder rounded once from the exact product.
-// The integer comes from the rounded product, so it may be off by its
-// rounding for very large angles (|dt A_imag| above 1e4, where the remainder
-// then exceeds 1/2 by that much: up to 2 steps at 1e5).
-__device__ __forceinline__ int angle_split_fine(float dt, float whb, float& r) {
-  const float kf = __builtin_rintf(fmul(dt, whb));
-  r = ffma(dt, whb, -kf);
-  int i;
-  // v_cvt_i32_f32 itself (it saturates; a C++ cast is undefined out of range)
-  asm("v_cvt_i32_f32 %0, %1" : "=v"(i) : "v"(kf));
-  return i & (kTabB - 1);
-}
-
-// whb: 2048 A_imag / (2 pi), the table's steps per unit of dt.
-__device__ __forceinline__ GatePartCS rot_gate_issue_cs(float dt, float pah, float whb, bool imag,
-                                                        const float2* tab) {
+__device__ __forceinline__ GatePartCS rot_gate_issue_cs(float dt, float pah, float wh, bool imag,
+                                                        const float2* cstab) {
   GatePartCS g;
   g.e = exp2_hw(fmul(dt, pah));
   if (!imag) {
@@ -461,22 +413,23 @@ __device__ __forceinline__ GatePartCS rot_gate_issue_cs(float dt, float pah, flo
     g.cs = make_float2(0.f, 0.f);
     return g;
   }
-  g.cs = tab[angle_split_fine(dt, whb, g.r)];
+  g.cs = cstab[angle_split(dt, wh, g.r)];
   return g;
 }
 
-// The gate e cos, and es = -a e sin (its derivative per table step).
 __device__ __forceinline__ float rot_gate_finish_cs(const GatePartCS& g, bool imag, float& es) {
   if (!imag) {
     es = 0.f;
     return g.e;
   }
-  const float r = g.r, am = fabsf(g.cs.x), t = g.cs.y;
-  const float p2 = ffma(-am, kC2B, kC2B);  // |cos| (-a^2 / 2)
-  const float u = ffma(r, p2, t);
-  const float w = ffma(r, u, -am);  // cos / b - 1 = -|m| + r (t + r p2)
-  // its derivative t (1 + kC2B r^2) + 2 r p2
-  const float v = ffma(r, ffma(r, fmul(t, kC2B), p2), u);
+  const float r = g.r, am = fabsf(g.cs.x), sb = g.cs.y;  // |m|, b sin
+  const float r2 = fmul(r, r);
+  const float cm1 = fmul(r2, kC2);                 // cos(a r) - 1
+  const float sx = fmul(r, ffma(r2, kS3, kS1));    // sin(a r)
+  // cos / b - 1 = cm1 - |m| (1 + cm1) - (b s) sin(a r)
+  const float w = ffma(-sb, sx, ffma(-am, cm1, cm1 - am));
+  // sin / b = (b s)(1 + cm1) + (1 - |m|) sin(a r)
+  const float v = ffma(sb, cm1, sb) + ffma(-am, sx, sx);
   const float be = signed_by(g.e, g.cs.x);
   es = fmul(be, v);
   return ffma(be, w, be);
@@ -537,9 +490,9 @@ __device__ __forceinline__ float gate_of(int j, int s, int NR, bool has_imag, fl
 // starts the rotational part of slot j, gate_finish_cs returns the gate.
 template <int S, class GK>
 __device__ __forceinline__ GatePartCS gate_issue_cs(int j, int NR, bool has_imag, float dt,
-                                                    float pah, float whb, const float2* tab) {
+                                                    float pah, float wh, const float2* cstab) {
   if (j >= GK::kTJ || (j >= GK::kRJ && j * S >= NR)) return GatePartCS{0.f, 0.f, {1.f, 0.f}};
-  return rot_gate_issue_cs(dt, pah, whb, imag_of<GK>(has_imag), tab);
+  return rot_gate_issue_cs(dt, pah, wh, imag_of<GK>(has_imag), cstab);
 }
 
 template <int S, class GK>

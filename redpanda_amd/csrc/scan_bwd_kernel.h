@@ -24,10 +24,10 @@
 // the backward walks chunks in reverse, recomputes the chunk's K steps into
 // registers (keeping s_{t-1}, the gate and e*sin, so the adjoint evaluates
 // no transcendental), then runs the adjoint over them.  The recompute
-// takes each gate and its sine from a finer table than the forward's (one
-// 8-byte read, a quadratic and its derivative: rp_device.h); each gate
-// matches the forward's to within an ulp and every chunk restarts from the
-// forward's checkpoint.
+// evaluates the forward's gate expansion from (m, b sin) table records,
+// which also give the sine (one 8-byte table read; the forward's records
+// would need a second read for it); each gate matches the forward's to
+// within an ulp and every chunk restarts from the forward's checkpoint.
 //
 // Streaming: the per-step inputs (dt, (dt*u)/2, u, dy per channel; B, C per
 // state) of a chunk and of the step before it sit in one of two LDS slots.
@@ -153,8 +153,8 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
   // wave's 32 distinct writes (DT channels x S / 2 pairs) meet distinct banks.
   constexpr int SP2 = S / 2, DDP = CB + DT;
   __shared__ float2 sDD[NB][K][SP2][DDP];
-  // (m, b (-s a)) records of the backward's gate table (none for real decay)
-  __shared__ float2 sCS[GK::kImag == 0 ? 1 : kTabB];
+  // (m, b sin) records of the gate table (none for real decay)
+  __shared__ float2 sCS[GK::kImag == 0 ? 1 : kTab];
   // per-thread float64 sums of the parameter gradients over the batch group
   // (dA_real or dtrack, dA_imag), kept in LDS to spare registers (in their
   // global partials when PAR_GLOBAL)
@@ -177,7 +177,7 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
   load_gate_regs<S, NPL>(gp, p.Ar, p.Ai, p.Tk, c, s, p.N, p.NR, p.NT, cvalid);
   // first read after the staging barrier below (the table stays from the
   // workgroup's first tile on)
-  if (GK::kImag != 0 && tpass == 0) fill_sincos_fine(sCS, tid);
+  if (GK::kImag != 0 && tpass == 0) fill_sincos_pairs(sCS, tid);
   // pam: the coefficient of the ddt sum over rotational states, zero for a
   // tracking state (only read for slots whose kind is decided at run time)
   float pam[NPL];
@@ -191,7 +191,6 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
 #pragma unroll
   for (int j = 0; j < NPL; ++j) {
     pam[j] = is_rot<S, GK>(j, s, p.NR) ? gp.pah[j] : 0.f;
-    gp.wh[j] *= (float)(kTabB / kTab);  // in the backward table's steps
     if constexpr (PAR_GLOBAL) {
       if (cvalid && j * S + s < p.N) {
         io.part_par[par_at(j)] = 0.0;
@@ -229,9 +228,12 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
   // sweep's (tile group, b) block of the dB / dC partials, pbc.
   uint32_t oDT[CPT], oU[CPT], oDY[CPT], oB[SPT], oC[SPT], oF[NFOLD][FPT], oD[DPT];
   uint32_t stDT = 0, stU = 0, stDY = 0, stB = 0, stC = 0, stF = 0;
-  // FAST: whether element k of this thread's channel-steps and state-steps
-  // exists (its place in the slot, its channel or state)
-  bool okC[CPT], okS[SPT], okD[DPT];
+  // FAST: the row (step of the slot, or of the chunk) of element k of this
+  // thread's channel-steps, state-steps and outputs, or kNone where it does not
+  // exist (its place in the slot, its channel or state): compared with the
+  // sequence's bounds, where a flag would hold a pair of scalar registers
+  constexpr int kNone = 1 << 30;
+  int rowC[CPT], rowS[SPT], rowD[DPT];
   float* pbc = io.part_bc;
   // FAST: fold output k of this thread as the LDS quad index of its wave-0
   // partials * 8 + its row within the fold, or -1 beyond the fold's outputs
@@ -264,7 +266,7 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
     for (int k = 0; k < CPT; ++k) {
       const int e = tid + k * kThreads;
       const int64_t t = t0 + sg * (e / CB - 1), c2 = tile * CB + e % CB;
-      okC[k] = e < KS * CB && c2 < p.D;
+      rowC[k] = e < KS * CB && c2 < p.D ? e / CB - 1 : kNone;
       oDT[k] = (uint32_t)((b * d_sb + t * d_sl + c2) * es_d) + word_off(dsrc);
       oU[k] = (uint32_t)((b * p.usb + t * p.usl + c2) * es_u) + word_off(p.u);
       oDY[k] = (uint32_t)((((int64_t)b * L + t) * p.D + c2) * 4);
@@ -274,7 +276,7 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
       const int e = tid + k * kThreads;
       const int kk = e % NP;
       const int64_t t = t0 + sg * (e / NP - 1), n = (kk % NPL) * S + kk / NPL;
-      okS[k] = e < KS * NP && n < p.N;
+      rowS[k] = e < KS * NP && n < p.N ? e / NP - 1 : kNone;
       oB[k] = (uint32_t)((b * p.bsb + t * p.bsl + n) * es_b) + word_off(p.Bc);
       oC[k] = (uint32_t)((b * p.csb + t * p.csl + n) * es_c) + word_off(p.Cc);
     }
@@ -293,7 +295,7 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
     for (int k = 0; k < DPT; ++k) {
       const int e = tid + k * kThreads;
       const int64_t t = t0 + sg * (e / CB), c2 = tile * CB + e % CB;
-      okD[k] = e < K * CB && c2 < p.D;
+      rowD[k] = e < K * CB && c2 < p.D ? e / CB : kNone;
       oD[k] = (uint32_t)((((int64_t)b * L + t) * p.D + c2) * 4);
     }
     stDT = (uint32_t)(sg * K * d_sl * es_d);
@@ -314,8 +316,8 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
   // is rotated to the word's low half by its byte offset (which keeps its
   // place in the word from chunk to chunk: K steps are a multiple of 8 bytes)
   // and shifted or converted.  A switch over the types' combinations cost its
-  // branches, and their joins' waits, in every chunk: at the Eval-Mamba shape
-  // 2.47 ms, 2.38 with words, 2.28 with the widths fixed.
+  // branches, and their joins' waits, in every chunk.  At the Eval-Mamba shape
+  // words take 2.37 ms and fixed widths 2.30 (fp32 2.36 and 2.26).
   using WDT = std::integral_constant<int, WD>;
   using WUT = std::integral_constant<int, WU>;
   auto load_el = [&](auto w_tag, const void* base, uint32_t off) -> uint32_t {
@@ -340,11 +342,10 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
       const uint32_t cu = (uint32_t)ch;
 #pragma unroll
       for (int k = 0; k < CPT; ++k) {
-        const int i = ch * K + (tid + k * kThreads) / CB - 1;
         rdt[k] = 0u;
         ru[k] = 0u;
         rdy[k] = 0.f;
-        if (okC[k] && (unsigned)i < (unsigned)L) {
+        if ((unsigned)(ch * K + rowC[k]) < (unsigned)L) {
           rdt[k] = load_el(WDT{}, dsrc, oDT[k] + cu * stDT);
           ru[k] = load_el(WUT{}, p.u, oU[k] + cu * stU);
           rdy[k] = load_byte<float>(io.dy, oDY[k] + cu * stDY);
@@ -352,10 +353,9 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
       }
 #pragma unroll
       for (int k = 0; k < SPT; ++k) {
-        const int i = ch * K + (tid + k * kThreads) / NP - 1;
         rb[k] = 0u;
         rc[k] = 0u;
-        if (okS[k] && (unsigned)i < (unsigned)L) {
+        if ((unsigned)(ch * K + rowS[k]) < (unsigned)L) {
           rb[k] = load_el(WDT{}, p.Bc, oB[k] + cu * stB);
           rc[k] = load_el(WDT{}, p.Cc, oC[k] + cu * stC);
         }
@@ -603,7 +603,7 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
             pdd[k][0] = 0.f;
             pdd[k][1] = 0.f;
             if constexpr (FAST) {
-              if (dir == 1 && okD[k] && (FULLC || (tid + k * kThreads) / CB < kcnt)) {
+              if (dir == 1 && rowD[k] < kcnt) {
                 const uint32_t o = oD[k] + (uint32_t)ch * stDY;
                 pdd[k][0] = load_byte<float>(io.pd_delta, o);
                 pdd[k][1] = load_byte<float>(io.pd_u, o);
@@ -732,7 +732,7 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
                   cpb[j] = ffma(t2, dt, cpb[j]);
                   if (j >= GK::kRJ) cpt[j] = cpt[j] + dg;
                   ddA = ffma(j < GK::kRJ ? gp.pah[j] : pam[j], t1, ddA);  // Ar log2(e) dg g
-                  ddB = ffma(gp.wh[j], t2, ddB);                          // -Ai dg e sin
+                  ddB = ffma(gp.wh[j], t2, ddB);                          // Ai 256/(2 pi) dg e sin
                 }
                 qn[j] = q;
                 gn[j] = g;
@@ -747,7 +747,8 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
               // rest of the sums over the channel's lanes are taken from sDD
               // at the chunk's end
               sDD[ONEBAR ? SL : 0][m][s / 2][cl] =
-                  make_float2(reduce_states<2>(ffma(kLn2, ddA, ddB)), reduce_states<2>(sBc));
+                  make_float2(reduce_states<2>(ffma(kLn2, ddA, -fmul(kRadPerStep, ddB))),
+                              reduce_states<2>(sBc));
               if constexpr (!FAST) fin = false;
             }
             if (m % KR == 0) {
@@ -830,7 +831,7 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
                 for (int k = 0; k < DPT; ++k) {
                   const int e = tid + k * kThreads;
                   if constexpr (FAST) {
-                    if (okD[k] && (FULL || e / CB < kcnt)) {
+                    if (rowD[k] < kcnt) {
                       const uint32_t o = oD[k] + (uint32_t)ch * stDY;
                       const float2 v = dd_of(ONEBAR ? SL : 0, e / CB, e % CB, fdt[k], fuh[k]);
                       float dd = dir == 0 ? v.x : pdd[k][0] + v.x;
@@ -881,12 +882,11 @@ __device__ __forceinline__ void scan_bwd_tile(const ScanParams& p, const BwdIO& 
                 if (cvalid && j * S + s < p.N) {
                   unsafeAtomicAdd(&io.part_par[par_at(j)], (double)a);
                   if (j < GK::kTJ)
-                    unsafeAtomicAdd(&io.part_par[par_at(j) + (int64_t)p.D * p.N],
-                                    (double)cpb[j] * kInvStepB);
+                    unsafeAtomicAdd(&io.part_par[par_at(j) + (int64_t)p.D * p.N], (double)cpb[j]);
                 }
               } else {
                 sPar[0][j][tid] += (double)a;
-                if (j < GK::kTJ) sPar[1][j][tid] += (double)cpb[j] * kInvStepB;
+                if (j < GK::kTJ) sPar[1][j][tid] += (double)cpb[j];
               }
               cpa[j] = 0.f;
               cpb[j] = 0.f;
