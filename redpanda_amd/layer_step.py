@@ -25,46 +25,63 @@ MAX_ROWS = 256
 
 
 def _plain_linear(m, out_features, in_features):
-    """A Linear of this shape that computes just that: no subclass,
-    parametrization or hook that a direct use of its weight would pass by."""
-    return (type(m) is nn.Linear and not m._forward_hooks and not m._forward_pre_hooks and
-            m.weight.shape == (out_features, in_features))
+    """The (tensor, shape) pairs of a Linear of this shape that computes just
+    that, or None: no subclass, parametrization or hook that a direct use of its
+    weight would pass by."""
+    if type(m) is not nn.Linear or m._forward_hooks or m._forward_pre_hooks:
+        return None
+    # (the dictionaries, not the attributes: this runs for every layer of a ply)
+    ps = m._parameters
+    pairs = [(ps.get("weight"), (out_features, in_features))]
+    if ps.get("bias") is not None:
+        pairs.append((ps["bias"], (out_features,)))
+    return pairs
+
+
+def _layer_tensors(layer, d):
+    """The (tensor, shape) pairs that hip_layer_step reads of a layer on rows of
+    d floats, or None where the separate ops must run."""
+    mx, norm = layer["mixer"], layer["norm"]
+    cfg = mx.config
+    D, r, np2 = cfg.d_inner, cfg.dt_rank, 2 * cfg.d_state * cfg.mimo_p
+    if cfg.d_model != d or d % 4 or D % 4 or r % 4 or cfg.mimo_p > 8:
+        return None
+    mods = mx._modules
+    pairs = [(norm.weight, (d,)), (mx.D, (D,))]
+    for name, n_out, n_in in (("in_proj", 2 * D, d), ("x_proj", r + np2, D), ("dt_proj", D, r),
+                              ("out_proj", d, D)):
+        lin = _plain_linear(mods.get(name), n_out, n_in)
+        if lin is None:
+            return None
+        pairs += lin
+    if cfg.use_bcnorm:
+        pairs += ((mx.b_norm.weight, (np2 // 2,)), (mx.c_norm.weight, (np2 // 2,)))
+    return pairs
 
 
 def usable(model, x):
     """Whether Mamba.step's inference loop may take hip_layer_step for the
-    rows x (R, d_model) fp32: a small batch, plain fp32 projections of the
-    configured shapes on x's device, contiguous and 16-byte aligned."""
-    cfg = model.config
-    d, D, r = cfg.d_model, cfg.d_inner, cfg.dt_rank
-    if x.shape[0] > MAX_ROWS or x.shape[0] == 0 or x.shape[1] != d or d % 4 or D % 4 or r % 4:
-        return False
-    if cfg.mimo_p > 8 or torch.is_autocast_enabled("cuda"):
+    rows x (R, d_model) fp32: a small batch, plain fp32 projections, and every
+    tensor of the configured shape, on x's device, contiguous and 16-byte
+    aligned (the kernels read them by these shapes; where one differs, the
+    separate ops refuse or convert it)."""
+    R, d = x.shape
+    if not 0 < R <= MAX_ROWS or torch.is_autocast_enabled("cuda"):
         return False
     if _nn_module._global_forward_hooks or _nn_module._global_forward_pre_hooks:
         return False
-    np2 = 2 * cfg.d_state * cfg.mimo_p
     dev = x.device
+    bits = 0
     for layer in model.layers:
-        mx = layer["mixer"]
-        if not (_plain_linear(mx.in_proj, 2 * D, d) and _plain_linear(mx.x_proj, r + np2, D) and
-                _plain_linear(mx.dt_proj, D, r) and _plain_linear(mx.out_proj, d, D)):
+        pairs = _layer_tensors(layer, d)
+        if pairs is None:
             return False
-        ws = [mx.in_proj.weight, mx.x_proj.weight, mx.dt_proj.weight, mx.out_proj.weight,
-              layer["norm"].weight, mx.D]
-        for lin in (mx.in_proj, mx.x_proj, mx.dt_proj, mx.out_proj):
-            if lin.bias is not None:
-                ws.append(lin.bias)
-        if cfg.use_bcnorm:
-            ws += (mx.b_norm.weight, mx.c_norm.weight)
-        bits = 0
-        for w in ws:
-            if w.dtype is not torch.float32 or w.device != dev or not w.is_contiguous():
+        for w, shape in pairs:
+            if (w is None or w.shape != shape or w.dtype is not torch.float32 or
+                    w.device != dev or not w.is_contiguous()):
                 return False
             bits |= w.data_ptr()
-        if bits & 15:
-            return False
-    return True
+    return not bits & 15
 
 
 def hip_layer_step(x, layer, state, compact=False, out=None):

@@ -1,0 +1,60 @@
+"""When Mamba.step takes the whole-layer call (redpanda_amd/layer_step.py):
+the models that must keep the separate ops, decided on the CPU from the models
+alone."""
+
+import pytest
+import torch
+import torch.nn as nn
+
+from redpanda_amd import layer_step
+from redpanda_amd.mamba import Mamba, MambaConfig
+
+
+def _model(**kw):
+    return Mamba(MambaConfig(**{**dict(d_model=64, n_layer=2, vocab_size=64, d_state=20,
+                                       n_track_state=4, mimo_p=2), **kw})).eval()
+
+
+def _x(R=4):
+    return torch.randn(R, 64)
+
+
+def _mixer(m):
+    return m.layers[1]["mixer"]
+
+
+def test_plain_models_take_it():
+    for kw in ({}, dict(bias=True), dict(use_bcnorm=False), dict(n_track_state=0),
+               dict(use_complex=False)):
+        assert layer_step.usable(_model(**kw), _x())
+
+
+@pytest.mark.parametrize("where,n", [
+    (lambda m: m.layers[1]["norm"], 1), (lambda m: m.layers[0]["norm"], 68),
+    (lambda m: _mixer(m).b_norm, 1), (lambda m: _mixer(m).c_norm, 44)])
+def test_norm_weights_of_another_length_are_left_to_the_separate_ops(where, n):
+    m = _model()
+    where(m).weight = nn.Parameter(torch.ones(n))
+    assert not layer_step.usable(m, _x())
+
+
+@pytest.mark.parametrize("proj", ["in_proj", "x_proj", "dt_proj", "out_proj"])
+def test_biases_of_another_length_are_left_to_the_separate_ops(proj):
+    m = _model(bias=True)
+    getattr(_mixer(m), proj).bias = nn.Parameter(torch.ones(4))
+    assert not layer_step.usable(m, _x())
+
+
+def test_a_skip_of_another_length_is_left_to_the_separate_ops():
+    m = _model()
+    _mixer(m).D = nn.Parameter(torch.ones(4))
+    assert not layer_step.usable(m, _x())
+
+
+def test_a_layer_is_judged_by_its_own_configuration():
+    """A mixer with BCNorm in a model configured without it."""
+    m = _model(use_bcnorm=False)
+    m.layers[1]["mixer"] = _model().layers[1]["mixer"]
+    assert layer_step.usable(m, _x())
+    _mixer(m).b_norm.weight = nn.Parameter(torch.ones(4))
+    assert not layer_step.usable(m, _x())
