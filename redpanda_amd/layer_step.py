@@ -14,7 +14,7 @@ import torch
 import torch.nn as nn
 from torch.nn.modules import module as _nn_module
 
-from redpanda_amd import _lib
+from redpanda_amd import _lib, mamba
 from redpanda_amd.step import _state_pair
 
 # Beyond this the separate launches, whose GEMMs then run at their own rate, were
@@ -24,11 +24,17 @@ from redpanda_amd.step import _state_pair
 MAX_ROWS = 256
 
 
+_LINEAR_FORWARD = nn.Linear.forward
+_PLAIN = (nn.Parameter, torch.Tensor)  # a tensor subclass computes its own product
+
+
 def _plain_linear(m, out_features, in_features):
     """The (tensor, shape) pairs of a Linear of this shape that computes just
-    that, or None: no subclass, parametrization or hook that a direct use of its
-    weight would pass by."""
-    if type(m) is not nn.Linear or m._forward_hooks or m._forward_pre_hooks:
+    that, or None: no subclass, parametrization, hook or forward of its own
+    (offloading and quantising wrappers set one on the instance) that a direct
+    use of its weight would pass by."""
+    if (type(m) is not nn.Linear or m._forward_hooks or m._forward_pre_hooks or
+            "forward" in m.__dict__):
         return None
     # (the dictionaries, not the attributes: this runs for every layer of a ply)
     ps = m._parameters
@@ -38,16 +44,23 @@ def _plain_linear(m, out_features, in_features):
     return pairs
 
 
+# what hip_layer_step does in Mamba3Block's place
+_BLOCK_METHODS = frozenset(("step", "_ssm_proj_raw"))
+
+
 def _layer_tensors(layer, d):
     """The (tensor, shape) pairs that hip_layer_step reads of a layer on rows of
     d floats, or None where the separate ops must run."""
     mx, norm = layer["mixer"], layer["norm"]
+    # a block whose step is not Mamba3Block's own has to run it
+    if type(mx) is not mamba.Mamba3Block or not _BLOCK_METHODS.isdisjoint(mx.__dict__):
+        return None
     cfg = mx.config
     D, r, np2 = cfg.d_inner, cfg.dt_rank, 2 * cfg.d_state * cfg.mimo_p
     if cfg.d_model != d or d % 4 or D % 4 or r % 4 or cfg.mimo_p > 8:
         return None
     mods = mx._modules
-    pairs = [(norm.weight, (d,)), (mx.D, (D,))]
+    pairs = [(norm._parameters.get("weight"), (d,)), (mx._parameters.get("D"), (D,))]
     for name, n_out, n_in in (("in_proj", 2 * D, d), ("x_proj", r + np2, D), ("dt_proj", D, r),
                               ("out_proj", d, D)):
         lin = _plain_linear(mods.get(name), n_out, n_in)
@@ -55,7 +68,8 @@ def _layer_tensors(layer, d):
             return None
         pairs += lin
     if cfg.use_bcnorm:
-        pairs += ((mx.b_norm.weight, (np2 // 2,)), (mx.c_norm.weight, (np2 // 2,)))
+        for name in ("b_norm", "c_norm"):
+            pairs.append((mods[name]._parameters.get("weight"), (np2 // 2,)))
     return pairs
 
 
@@ -70,6 +84,8 @@ def usable(model, x):
         return False
     if _nn_module._global_forward_hooks or _nn_module._global_forward_pre_hooks:
         return False
+    if nn.Linear.forward is not _LINEAR_FORWARD or mamba.Mamba3Block.step is not mamba._BLOCK_STEP:
+        return False  # replaced for every instance
     dev = x.device
     bits = 0
     for layer in model.layers:
@@ -77,7 +93,7 @@ def usable(model, x):
         if pairs is None:
             return False
         for w, shape in pairs:
-            if (w is None or w.shape != shape or w.dtype is not torch.float32 or
+            if (type(w) not in _PLAIN or w.shape != shape or w.dtype is not torch.float32 or
                     w.device != dev or not w.is_contiguous()):
                 return False
             bits |= w.data_ptr()

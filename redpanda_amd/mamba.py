@@ -348,6 +348,9 @@ class Mamba3Block(nn.Module):
         return self.out_proj(y), (h, beta)
 
 
+_BLOCK_STEP = Mamba3Block.step  # (layer_step.py tells a replaced one by it)
+
+
 class Mamba(nn.Module):
     """Embedding + n_layer pre-norm Mamba-3 blocks + final norm (engine/mamba.py:503-620)."""
 

@@ -7,7 +7,7 @@ import torch
 import torch.nn as nn
 
 from redpanda_amd import layer_step
-from redpanda_amd.mamba import Mamba, MambaConfig
+from redpanda_amd.mamba import Mamba, Mamba3Block, MambaConfig
 
 
 def _model(**kw):
@@ -58,3 +58,56 @@ def test_a_layer_is_judged_by_its_own_configuration():
     assert layer_step.usable(m, _x())
     _mixer(m).b_norm.weight = nn.Parameter(torch.ones(4))
     assert not layer_step.usable(m, _x())
+
+
+class _CountingBlock(Mamba3Block):
+    def step(self, *args, **kw):
+        return super().step(*args, **kw)
+
+
+def _subclass(m, monkeypatch):
+    _mixer(m).__class__ = _CountingBlock
+
+
+def _own_step(m, monkeypatch):
+    block = _mixer(m)
+    block.step = lambda *args, **kw: Mamba3Block.step(block, *args, **kw)
+
+
+def _class_step(m, monkeypatch):
+    step = Mamba3Block.step
+    monkeypatch.setattr(Mamba3Block, "step", lambda self, *args, **kw: step(self, *args, **kw))
+
+
+def _own_forward(m, monkeypatch):
+    lin = _mixer(m).dt_proj
+    lin.forward = lambda x: nn.Linear.forward(lin, x) * 2
+
+
+def _class_forward(m, monkeypatch):
+    fwd = nn.Linear.forward
+    monkeypatch.setattr(nn.Linear, "forward", lambda self, x: fwd(self, x) * 2)
+
+
+class _Wrapped(torch.Tensor):
+    pass
+
+
+def _tensor_subclass(m, monkeypatch):
+    lin = _mixer(m).in_proj
+    lin.weight = nn.Parameter(lin.weight.detach().as_subclass(_Wrapped))
+
+
+def _no_module(m, monkeypatch):
+    _mixer(m).x_proj = nn.Sequential(_mixer(m).x_proj)
+
+
+@pytest.mark.parametrize("change", [_subclass, _own_step, _class_step, _own_forward, _class_forward,
+                                    _tensor_subclass, _no_module])
+def test_replaced_methods_and_types_keep_the_separate_ops(change, monkeypatch):
+    """What ran in the layer's place before the whole-layer call still runs."""
+    m = _model()
+    change(m, monkeypatch)
+    assert not layer_step.usable(m, _x())
+    monkeypatch.undo()
+    assert layer_step.usable(_model(), _x())
