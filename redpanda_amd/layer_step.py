@@ -100,6 +100,23 @@ def usable(model, x):
     return not bits & 15
 
 
+def _vector_rows(x):
+    """(tensor, row stride): the rows of x (R, d) where the kernels can read
+    them as 16-byte vectors, x itself or a copy.  (contiguous() would return a
+    misaligned x, or one row of another stride, as it is.)  A stride shorter
+    than a row is left to the library, which refuses it."""
+    R, d = x.shape
+    if x.stride(-1) != 1:
+        x = x.contiguous()
+    sr = x.stride(0)
+    if sr >= d:
+        if R == 1:
+            sr = d
+        if sr % 4 or x.data_ptr() & 15:
+            x, sr = torch.empty((R, d), dtype=x.dtype, device=x.device).copy_(x), d
+    return x, sr
+
+
 def hip_layer_step(x, layer, state, compact=False, out=None):
     """(x + layer(x), (h, beta)) for rows x (R, d_model) fp32 that `usable`
     accepted; state, compact and out as in Mamba3Block.step."""
@@ -108,8 +125,7 @@ def hip_layer_step(x, layer, state, compact=False, out=None):
     cfg = mx.config
     R, D, N = x.shape[0], cfg.d_inner, cfg.d_state
     dev = x.device
-    if x.stride(-1) != 1 or x.stride(0) % 4 or x.data_ptr() & 15:
-        x = x.contiguous()
+    x, x_sr = _vector_rows(x)
     Ar, Ai, Tk = mx._gates(False)
     a = _lib.LayerStepArgs()
     a.R, a.d_model, a.D, a.N = R, cfg.d_model, D, N
@@ -131,7 +147,7 @@ def hip_layer_step(x, layer, state, compact=False, out=None):
                 raise ValueError(f"step: out {name} must be a contiguous fp32 {shp} tensor on {dev}")
     x_out = torch.empty((R, cfg.d_model), **f32)
     norm = layer["norm"]
-    a.x, a.x_sr, a.norm_w, a.norm_eps = x.data_ptr(), x.stride(0), norm.weight.data_ptr(), norm.eps
+    a.x, a.x_sr, a.norm_w, a.norm_eps = x.data_ptr(), x_sr, norm.weight.data_ptr(), norm.eps
     for pre, lin in (("in", mx.in_proj), ("xp", mx.x_proj), ("dtp", mx.dt_proj), ("out", mx.out_proj)):
         setattr(a, pre + "_w", lin.weight.data_ptr())
         if lin.bias is not None:
