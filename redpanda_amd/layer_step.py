@@ -15,7 +15,7 @@ import torch.nn as nn
 from torch.nn.modules import module as _nn_module
 
 from redpanda_amd import _lib, mamba
-from redpanda_amd.step import _state_pair
+from redpanda_amd.step import _f32c, _state_pair
 
 # Beyond this the separate launches, whose GEMMs then run at their own rate, were
 # not measured against it: at 8 layers of d_model 512, 12 / 64 / 256 rows, an
@@ -117,6 +117,20 @@ def _vector_rows(x):
     return x, sr
 
 
+def _gate_rows(gates, D, N):
+    """(A_real, A_imag, track) as fp32 rows of the D channels: the parameters
+    they come from may be views of any stride, which the gates keep."""
+    Ar, Ai, Tk = (None if t is None else _f32c(t) for t in gates)
+    NR = 0 if Ar is None else Ar.shape[-1]
+    NT = 0 if Tk is None else Tk.shape[-1]
+    if NR + NT != N:
+        raise ValueError(f"step: n_rot ({NR}) + n_track ({NT}) != d_state ({N})")
+    for t, n in ((Ar, NR), (Ai, NR), (Tk, NT)):
+        if t is not None and t.shape != (D, n):
+            raise ValueError(f"step: gates {tuple(t.shape)} must be {(D, n)}")
+    return Ar, Ai, Tk
+
+
 def hip_layer_step(x, layer, state, compact=False, out=None):
     """(x + layer(x), (h, beta)) for rows x (R, d_model) fp32 that `usable`
     accepted; state, compact and out as in Mamba3Block.step."""
@@ -126,10 +140,11 @@ def hip_layer_step(x, layer, state, compact=False, out=None):
     R, D, N = x.shape[0], cfg.d_inner, cfg.d_state
     dev = x.device
     x, x_sr = _vector_rows(x)
-    Ar, Ai, Tk = mx._gates(False)
+    Ar, Ai, Tk = _gate_rows(mx._gates(False), D, N)
     a = _lib.LayerStepArgs()
-    a.R, a.d_model, a.D, a.N = R, cfg.d_model, D, N
-    a.NR, a.NT, a.P, a.dt_rank = cfg.n_rot_state, cfg.n_track_state, cfg.mimo_p, cfg.dt_rank
+    a.R, a.d_model, a.D, a.N, a.P, a.dt_rank = R, cfg.d_model, D, N, cfg.mimo_p, cfg.dt_rank
+    a.NR = 0 if Ar is None else Ar.shape[1]
+    a.NT = 0 if Tk is None else Tk.shape[1]
     h_in = beta_in = None
     rank1 = bool(compact)
     if state is not None:
