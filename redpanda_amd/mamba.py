@@ -412,7 +412,7 @@ class Mamba(nn.Module):
             x.requires_grad or any(p.requires_grad for p in self.parameters()) or
             any(t.requires_grad for st in cache if st is not None for t in st))
         if not record and x.dtype == torch.float32 and x.dim() == 2 and len(self.layers) > 0:
-            if layer_step.usable(self, x):
+            if x.is_cuda and layer_step.usable(self, x):
                 # a small batch of plain fp32 layers: one library call each
                 for i, layer in enumerate(self.layers):
                     x, st = layer_step.hip_layer_step(x, layer, cache[i], compact=compact,

@@ -111,3 +111,9 @@ def test_replaced_methods_and_types_keep_the_separate_ops(change, monkeypatch):
     assert not layer_step.usable(m, _x())
     monkeypatch.undo()
     assert layer_step.usable(_model(), _x())
+
+
+def test_host_tensors_are_refused_as_before():
+    """By the separate ops' own check, whether or not a GPU is there."""
+    with torch.no_grad(), pytest.raises(ValueError, match="device tensor"):
+        _model().step(input_embed=_x())
