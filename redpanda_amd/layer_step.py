@@ -17,11 +17,27 @@ from torch.nn.modules import module as _nn_module
 from redpanda_amd import _lib, mamba
 from redpanda_amd.step import _f32c, _state_pair
 
-# Beyond this the separate launches, whose GEMMs then run at their own rate, were
-# not measured against it: at 8 layers of d_model 512, 12 / 64 / 256 rows, an
-# eager ply takes 0.50 / 0.49 / 0.58 ms against 1.32 / 1.32 / 1.35, a replayed
-# one 0.27 / 0.30 / 0.57 against 0.40 / 0.44 / 0.60.
+# The most rows that take this path, by width (d_model, at expand 2).  A
+# projection's workgroup here reads all of its x rows for 16 columns of W, which
+# costs more than its launch saves once rows and width grow; the library's GEMMs
+# share both in larger tiles.  Microseconds per layer of a replayed ply, this path / the separate ops
+# (eager: the larger of this and the host's 48 / 150):
+#   d_model  256   64 rows 25 / 74,  256 35 / 200,  512 56 / 63
+#   d_model  512   64 34 / 51,  256 64 / 67,  384 87 / 78
+#   d_model  640   128 65 / 66,  144 65 / 63,  256 93 / 81
+#   d_model  768   64 47 / 53,  128 72 / 72,  144 79 / 68,  256 105 / 88
+#   d_model 1024   64 53 / 63,  128 82 / 85,  144 104 / 88,  256 130 / 105
+#   d_model 1280   48 73 / 75,  64 93 / 89
+#   d_model 1536   32 76 / 87,  48 99 / 96,  128 151 / 125
+#   d_model 2048   32 100 / 108,  48 119 / 118,  128 209 / 159,  256 374 / 239
+# (Replayed and eager plies take the same path, so that they give the same bits.)
 MAX_ROWS = 256
+
+
+def max_rows(width):
+    if width <= 512:
+        return MAX_ROWS
+    return MAX_ROWS // 2 if width <= 1024 else min(MAX_ROWS // 2, (1 << 16) // width)
 
 
 _LINEAR_FORWARD = nn.Linear.forward
@@ -75,12 +91,13 @@ def _layer_tensors(layer, d):
 
 def usable(model, x):
     """Whether Mamba.step's inference loop may take hip_layer_step for the
-    rows x (R, d_model) fp32: a small batch, plain fp32 projections, and every
+    rows x (R, d_model) fp32: a small batch for the width, plain fp32 projections, and every
     tensor of the configured shape, on x's device, contiguous and 16-byte
     aligned (the kernels read them by these shapes; where one differs, the
     separate ops refuse or convert it)."""
     R, d = x.shape
-    if not 0 < R <= MAX_ROWS or torch.is_autocast_enabled("cuda"):
+    if (not 0 < R <= max_rows(max(d, model.config.d_inner // 2)) or
+            torch.is_autocast_enabled("cuda")):
         return False
     if _nn_module._global_forward_hooks or _nn_module._global_forward_pre_hooks:
         return False

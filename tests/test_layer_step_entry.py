@@ -117,3 +117,17 @@ def test_host_tensors_are_refused_as_before():
     """By the separate ops' own check, whether or not a GPU is there."""
     with torch.no_grad(), pytest.raises(ValueError, match="device tensor"):
         _model().step(input_embed=_x())
+
+
+@pytest.mark.parametrize("d,rows", [(64, 256), (512, 256), (576, 128), (1024, 128), (1280, 51),
+                                    (2048, 32)])
+def test_the_most_rows_fall_with_the_width(d, rows):
+    m = _model(d_model=d, n_layer=1)
+    assert layer_step.usable(m, torch.zeros(rows, d))
+    assert not layer_step.usable(m, torch.zeros(rows + 1, d))
+
+
+def test_the_inner_width_counts_too():
+    m = _model(d_model=256, expand=8, n_layer=1)  # as wide as d_model 1024
+    assert layer_step.usable(m, torch.zeros(128, 256))
+    assert not layer_step.usable(m, torch.zeros(129, 256))
