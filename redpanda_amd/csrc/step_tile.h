@@ -130,21 +130,6 @@ __global__ __launch_bounds__(kThreads) void step_tile_kernel(StepParams p) {
   const bool has_imag = p.Ai != nullptr;
   const int r_lo = rg * p.ri;
   const int nr = min(p.R, r_lo + p.ri) - r_lo;  // <= RIM (checked by the host)
-  // a rollout's block of the input state: its own, or the one shared state
-  // (ssr == 0)
-  auto load_block = [&](int64_t r, float4 (&hl)[NB], float4 (&bl)[NB]) {
-    const int64_t iblk = r * (p.ssr / 4) + (int64_t)c0 * NVM;
-    const float4* hi4 = reinterpret_cast<const float4*>(p.h_in) + iblk;
-    const float4* bi4 = reinterpret_cast<const float4*>(p.beta_in) + iblk;
-#pragma unroll
-    for (int m = 0; m < NB; ++m) {
-      const int k = tid + m * kThreads;
-      if ((FULLD && !PAD && WHOLE) || k < nvalid) {
-        hl[m] = SHARED ? hi4[k] : load_stream(hi4 + k);
-        if constexpr (!RANK1) bl[m] = SHARED ? bi4[k] : load_stream(bi4 + k);
-      }
-    }
-  };
   // ONE: the rollout's inputs, ahead of the prologue's loads
   float dt1 = 0.f, u1 = 0.f, z1 = 0.f, dtup1 = 0.f;
   float4 h1[ONE ? NB : 1], b1[ONE ? NB : 1];
@@ -154,7 +139,17 @@ __global__ __launch_bounds__(kThreads) void step_tile_kernel(StepParams p) {
     if (p.z != nullptr) z1 = load_in(p.z, (int64_t)r_lo * p.zsr + cld, p.dt_z);
     if (p.h_in != nullptr) {
       if constexpr (RANK1) dtup1 = p.beta_in[(int64_t)r_lo * p.bssr + cld];
-      load_block(r_lo, h1, b1);
+      const int64_t iblk = r_lo * (p.ssr / 4) + (int64_t)c0 * NVM;
+      const float4* hi4 = reinterpret_cast<const float4*>(p.h_in) + iblk;
+      const float4* bi4 = reinterpret_cast<const float4*>(p.beta_in) + iblk;
+#pragma unroll
+      for (int m = 0; m < NB; ++m) {
+        const int k = tid + m * kThreads;
+        if ((FULLD && !PAD && WHOLE) || k < nvalid) {
+          h1[m] = load_stream(hi4 + k);
+          if constexpr (!RANK1) b1[m] = load_stream(bi4 + k);
+        }
+      }
     }
   }
   // The prologue issues every load (B / C rows, gate parameters, D) before
@@ -190,8 +185,11 @@ __global__ __launch_bounds__(kThreads) void step_tile_kernel(StepParams p) {
   // and 10.0 -> 6.8 at 64 (D 1024, 16 + 4 states), 262 -> 254 at 4096; rank-1
   // rows 43 -> 33 at 777 and 149 -> 136 at 4096.  Not with 16 slices, the full
   // beta and several rollouts per workgroup: there the scalar form stays (64
-  // states, 4096 rollouts: 780 us, 819 with vectors).
-  constexpr bool VEC = S != 16 || RANK1 || ONE;
+  // states, 4096 rollouts: 780 us, 819 with vectors), and likewise with rank-1
+  // rows and pad states above 4 slots (28 + 8 states 261 us, 270 with vectors;
+  // 64 + 8 548 and 557, 100 + 8 800 and 822; up to 4 slots vectors are 3-9 %
+  // faster: 24 + 4 208 -> 190, 56 + 4 475 -> 462).
+  constexpr bool VEC = ONE || (RANK1 ? !PAD || NPL <= 4 : S != 16);
   if (VEC && p.gate_vec) {
 #pragma unroll
     for (int v = 0; v < NVT; ++v) {
@@ -266,7 +264,24 @@ __global__ __launch_bounds__(kThreads) void step_tile_kernel(StepParams p) {
     if constexpr (!ONE) zz = p.z != nullptr ? load_in(p.z, r * p.zsr + cld, p.dt_z) : 0.f;
     // rank-1: the channel's (dt*u)_prev, halved as the scan halves dt*u
     float hdp = 0.f;
-    auto store_block = [&](const float4 (&hl)[NB], const float4 (&bl)[NB]) {
+    if (p.h_in != nullptr) {
+      if constexpr (RANK1) hdp = 0.5f * (ONE ? dtup1 : p.beta_in[r * p.bssr + cld]);
+      // input block: the rollout's own, or the one shared state (ssr == 0)
+      const int64_t iblk = r * (p.ssr / 4) + (int64_t)c0 * NVM;
+      const float4* hi4 = reinterpret_cast<const float4*>(p.h_in) + iblk;
+      const float4* bi4 = reinterpret_cast<const float4*>(p.beta_in) + iblk;
+      float4 hl[NB], bl[NB];
+#pragma unroll
+      for (int m = 0; m < NB; ++m) {
+        const int k = tid + m * kThreads;
+        if constexpr (ONE) {
+          hl[m] = h1[m];
+          bl[m] = b1[m];
+        } else if ((FULLD && !PAD && WHOLE) || k < nvalid) {
+          hl[m] = SHARED ? hi4[k] : load_stream(hi4 + k);
+          if constexpr (!RANK1) bl[m] = SHARED ? bi4[k] : load_stream(bi4 + k);
+        }
+      }
 #pragma unroll
       for (int m = 0; m < NB; ++m) {
         const int k = tid + m * kThreads;
@@ -274,17 +289,6 @@ __global__ __launch_bounds__(kThreads) void step_tile_kernel(StepParams p) {
           sH[k] = hl[m];
           if constexpr (!RANK1) sBt[k] = bl[m];
         }
-      }
-    };
-    if (p.h_in != nullptr) {
-      if constexpr (ONE) {
-        if constexpr (RANK1) hdp = 0.5f * dtup1;
-        store_block(h1, b1);
-      } else {
-        if constexpr (RANK1) hdp = 0.5f * p.beta_in[r * p.bssr + cld];
-        float4 hl[NB], bl[NB];
-        load_block(r, hl, bl);
-        store_block(hl, bl);
       }
     } else {
 #pragma unroll
