@@ -305,8 +305,7 @@ def test_backward_tile_walk_matches_single_tile(gpu_lib, D, bidir):
     are independent, so every checked row of the large batch has the
     single-row run's bits in y, d_delta and d_u (per-channel sums), and its
     dB / dC within about one fp32 rounding per tile (their partials are added
-    in another order).  D=120 leaves a partial tile: the general
-    instantiation walks too."""
+    in another order).  D=120 leaves a partial tile."""
     B, L, NR, NT = 1100, 9, 64, 8
     c = make_case(808, B=B, L=L, D=D, NR=NR, NT=NT)
     y, g = hip_capi.scan_fwd_bwd(c, bidir)
@@ -400,7 +399,7 @@ def test_final_state_gradients(gpu_lib):
         assert e <= 2e-6, f"{k}: {e:.3e}"
 
 
-# ─── whole-tile fast paths against the partial-tile path, bit for bit ───────
+# ─── whole channel tiles against partial ones, bit for bit ─────────────────
 
 def _lanes_per_channel(N):
     return 4 if N <= 20 else (8 if N <= 40 else 16)
@@ -422,9 +421,8 @@ STORAGE = {
 @pytest.mark.parametrize("bidir", [False, True])
 def test_whole_tile_paths_equal_partial_tile(gpu_lib, N, NT, storage, bidir):
     """Channels are independent, so a launch over D = CB channels (one whole
-    tile: the forward's fast staging of full blocks, and the backward's
-    whole-tile instantiation) and one over D = CB - 1 (a partial tile: the
-    element-wise staging and the general backward) must give the first CB - 1
+    tile) and one over D = CB - 1 (a partial tile, whose missing channel's
+    lanes stage zeros and store nothing) must give the first CB - 1
     channels the same bits: y; for causal scans the final state; d_delta,
     d_u and the parameter gradients, each a per-channel sum in a fixed order
     (dB / dC sum over channels and are left out).  L = 70 covers full blocks
