@@ -135,6 +135,8 @@ def hip_step(delta, u, Bc, Cc, A_real, A_imag, track, Dskip, state=None, out=Non
         B_raw, C_raw, wB, wC, P, eps, normalize = bcnorm
         if B_raw.shape != C_raw.shape or B_raw.shape[0] != R or B_raw.shape[-1] % P:
             raise ValueError(f"step: bcnorm projections must be (R, N * P) = ({R}, N * {P})")
+        if normalize and (wB.numel() != B_raw.shape[-1] or wC.numel() != B_raw.shape[-1]):
+            raise ValueError(f"step: BCNorm's weights must be ({B_raw.shape[-1]},)")
         Bx, Cx = _bn_rows(B_raw), _bn_rows(C_raw)
         if Cx.dtype != Bx.dtype:
             Cx = Cx.to(Bx.dtype)
@@ -151,6 +153,10 @@ def hip_step(delta, u, Bc, Cc, A_real, A_imag, track, Dskip, state=None, out=Non
         raise ValueError(f"step: n_rot ({NR}) + n_track ({NT}) != d_state ({N})")
     if delta.shape != (R, D) or Bc.shape != (R, N) or Cc.shape != (R, N):
         raise ValueError("step: delta/u must be (R, D) and B/C (R, N)")
+    # (read by these sizes, whatever the tensors hold)
+    for t, n in ((A_real, D * NR), (A_imag, D * NR), (track, D * NT), (Dskip, D)):
+        if t is not None and t.numel() != n:
+            raise ValueError(f"step: {tuple(t.shape)} must hold {n} values for D = {D} channels")
     dev = u.device
     delta, u, Bc, Cc = (_rows(t) for t in (delta, u, Bc, Cc))
     Ar = None if A_real is None else _f32c(A_real)
