@@ -451,7 +451,9 @@ int rp_step_bcnorm(const rp_step_args* a, const rp_bcnorm_args* bn, void* stream
 /*
  * One layer of the inference step in fp32, whole: the pre-norm, the
  * projections, the step and the residual add of Mamba.step's loop
- * (engine/mamba.py:440-498 and :592-597), as five launches from one call:
+ * (engine/mamba.py:440-498 and :592-597), as five launches from one call
+ * (six where BCNorm takes one of its own: several rollouts per workgroup of the
+ * step, or more than 64 states):
  *   in_proj of norm(x) (SiLU on its first D outputs), x_proj, dt_proj,
  *   rp_step_bcnorm (gated by z), x_out = x + out_proj.
  * For small batches, where a layer is launches and latency: x is (R,

@@ -425,8 +425,11 @@ __global__ __launch_bounds__(kThreads, (fwd_bound<S, NPL, FEW>())) void scan_fwd
   }
 }
 
-// The types that small launches come in have the FEW instantiations: fp32 and
-// the model's.
+// The types that small launches come in have the FEW instantiations: fp32, bf16
+// and the model's.  Plain fp16, the autocast mix and the run-time mix would gain
+// by it as well (B 1, L 67, D 768, N 32: 28 / 28 / 31 us, 21 / 21 / 25 with FEW;
+// B 32, L 64, D 1024: 41 / 42 / 45 and 40 / 40 / 40); they have none to keep the
+// library smaller by 2.3 MB.
 constexpr bool fwd_has_few(int TY) {
   return TY == kFwdF32 || TY == kFwdBf16 || TY == kFwdF32Sp || TY == kFwdModelBf16 ||
          TY == kFwdModelF16;

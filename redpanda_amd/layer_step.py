@@ -3,9 +3,9 @@
 `hip_layer_step` is the body of Mamba.step's pre-norm loop for one layer
 (engine/mamba.py:592-597 around Mamba3Block.step, :440-498): x + out_proj of
 the gated step of norm(x), with the norm, SiLU and residual add folded into
-small-batch fp32 projections (rp_layer_step: five launches where the separate
-ops take seven, and one call from Python where they take eight).  Inference
-only.
+small-batch fp32 projections (rp_layer_step: five launches, six where BCNorm does
+not fit the step's prologue, where the separate ops take seven and eight, and one
+call from Python where they take eight).  Inference only.
 """
 
 import ctypes

@@ -2,12 +2,12 @@
 
 At the rollout counts MARS runs (survivors x simulations, a few to a few
 hundred rows: engine/mars_search.py:59, :440-449), one Mamba.step ply is
-bound by the host: each of the n_layer layers issues five launches from one
-call (layer_step.py; seven from eight above 256 rows or where that path does
-not apply), about 0.5 ms per ply for 8 layers up to 128 rows (1.3 ms),
-against 11-28 us of step kernel per layer.  StepGraph records one ply of
+bound by the host: each of the n_layer layers issues five or six launches from
+one call (layer_step.py), about 0.43 ms per ply for 8 layers of d_model 512 up
+to 128 rows, or seven from eight where that path does not apply (1.3 ms),
+against 5-11 us of step kernel per layer.  StepGraph records one ply of
 Mamba.step for a fixed batch once and replays it: every launch of the ply is
-issued by one graph launch (0.27 ms at 12 rows, 0.30 at 64).
+issued by one graph launch (0.21 ms at 1 row, 0.25 at 32, 0.33 at 128).
 
 The state lives in two static cache sets that the two captured graphs use in
 turn (graph 0 reads set 0 and writes set 1, graph 1 the reverse), so a ply

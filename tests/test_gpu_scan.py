@@ -274,9 +274,8 @@ def test_backward_is_deterministic(gpu_lib):
                                      (120, 8, 48)])
 @pytest.mark.parametrize("softplus", [False, True])
 def test_whole_tile_backward_equals_general(gpu_lib, NR, NT, D, softplus):
-    """The backward's whole-tile instantiation (no initial state, no final-state
-    gradients, D a multiple of the tile) against its general one on the same
-    causal scan, taken by passing an all-zero initial state and all-zero
+    """The backward's FAST instantiation (no initial state, no final-state
+    gradients) against its general one on the same causal scan, taken by passing an all-zero initial state and all-zero
     final-state gradients: every output bit for bit (L=37 ends in a partial
     chunk).  The state counts cover every lane split (4, 8 and 16 lanes per
     channel, 1 to 8 states per lane, padded slots) and so every way the
