@@ -154,9 +154,9 @@ def hip_step(delta, u, Bc, Cc, A_real, A_imag, track, Dskip, state=None, out=Non
     if delta.shape != (R, D) or Bc.shape != (R, N) or Cc.shape != (R, N):
         raise ValueError("step: delta/u must be (R, D) and B/C (R, N)")
     # (read by these sizes, whatever the tensors hold)
-    for t, n in ((A_real, D * NR), (A_imag, D * NR), (track, D * NT), (Dskip, D)):
-        if t is not None and t.numel() != n:
-            raise ValueError(f"step: {tuple(t.shape)} must hold {n} values for D = {D} channels")
+    if (Dskip.numel() != D or (NR and A_real.numel() != D * NR) or (NT and track.numel() != D * NT) or
+            (A_imag is not None and A_imag.numel() != D * NR)):
+        raise ValueError(f"step: the gates and the skip must hold their values for D = {D} channels")
     dev = u.device
     delta, u, Bc, Cc = (_rows(t) for t in (delta, u, Bc, Cc))
     Ar = None if A_real is None else _f32c(A_real)
